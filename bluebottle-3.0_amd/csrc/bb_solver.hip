@@ -144,6 +144,7 @@ struct CGState {
   double rz_ref;      /* mixed form: (r, z) at the last FP64 correction */
   double relup;       /* mixed form: inner reduction of (r, z) per sweep */
   int q, done, nan_flag, inner_done;
+  int lost;           /* a one-launch sweep gave up waiting */
   double alpha;       /* alpha of the last update that left phi alone */
 };
 
@@ -236,6 +237,7 @@ cg_state_init_kernel(const double *__restrict__ bpart,
     st->done = 0;
     st->nan_flag = 0;
     st->inner_done = 0;
+    st->lost = 0;
     st->alpha = 0.;
   }
 }
@@ -1422,6 +1424,8 @@ update_row_kernel(DevDom D, InvMT<V> T, CGState *st, int q,
   }
 }
 
+#include "bb_resident.h"
+
 /* Every 50th iteration (src/cuda_solver.cu:208-224): phi += alpha p ... */
 __global__ void __launch_bounds__(TILE_THREADS)
 update_solution_kernel(DevDom D, const CGState *st, int q,
@@ -1988,13 +1992,17 @@ mx_residual_kernel(DevDom D, Coef K, InvMTab T, const double *__restrict__ phi,
  * it becomes the reference for the next inner sweep.  With `restart` the
  * next iteration q + 1 starts a fresh Krylov space (classic defect
  * correction); otherwise the search direction is kept and beta is formed
- * from the FP64 value by the next search launch (a reliable update). */
+ * from the FP64 value by the next search launch (a reliable update).
+ * q < 0: the sweep ran in one launch and left its length in the state (and
+ * where it ran out of iterations, there is nothing to decide). */
 __global__ void __launch_bounds__(TILE_THREADS)
 mx_state_kernel(CGState *st, const double *__restrict__ rpart, long n, int q,
   int restart)
 {
+  if (q < 0 && (st->lost || !st->inner_done)) return;
   double s = tile_block_sum(rpart, n);
   if (threadIdx.x != 0) return;
+  if (q < 0) q = st->q;
   st->rz1 = s;
   if (s <= st->tol2*st->sp_rhs || isnan(s)) {
     st->done = 1;
@@ -2045,6 +2053,10 @@ static double *_part_p = NULL;         /* tile partials of (p, Ap) */
 static double *_part_r = NULL;         /* tile partials of (r, z) */
 static double *_part_w1 = NULL, *_part_w2 = NULL;  /* learned-guess scale */
 static long buf_n = 0, part_n = 0;
+static u64 *_meet = NULL;              /* slots of the one-launch sweep */
+static int resident_cus = 0;           /* CUs of the device; -1: not used any
+                                          more (it could not be launched, or
+                                          gave up waiting) */
 int bb_pcg_batch = 16;                 /* iterations enqueued per host check */
 int bb_pcg_predict = 1;                /* 1: the first check of a sweep comes
                                           after 0.8 of the length the same
@@ -2154,6 +2166,13 @@ int bb_spmv_tzb32 = 0;                 /* tiles per z-column of the FP32
 int bb_defer_phi = 1;                  /* 1: phi updated every second
                                           iteration with both terms */
 int bb_mixed_restart = 0;              /* 1: restart CG at every correction */
+int bb_resident = 1;                   /* 1: grids that fit run a whole sweep
+                                          in one launch (bb_resident.h); 0:
+                                          two kernels per iteration always */
+int bb_resident_spins = 1 << 21;       /* polls (about a microsecond each)
+                                          before a wait in it gives up */
+int bb_resident_last = 0;              /* tiles per workgroup of the last
+                                          sweep, 0: kernel by kernel */
 long bb_pcg_iters_total = 0;           /* PCG iterations over all solves */
 long bb_pcg_solves_total = 0;
 /* Iterations of each solve, in order (entry n % BB_SOLVE_LOG of solve n). */
@@ -2236,6 +2255,9 @@ void bb_solver_free(void)
   if (_cg_state) BB_CHECK(hipFree(_cg_state));
   if (cg_host) BB_CHECK(hipHostFree(cg_host));
   cg_buffers32_free();
+  if (_meet) BB_CHECK(hipFree(_meet));
+  _meet = NULL;
+  resident_cus = 0;
   _cg_state = NULL;
   cg_host = NULL;
   _p_alt = _part_p = _part_r = NULL;
@@ -2840,6 +2862,89 @@ static void enqueue_iteration(int q, const Coef &K, const InvMTab &T)
   BB_LAUNCH_CHECK();
 }
 
+/* Tiles per workgroup of the one-launch sweep with vectors of `esize` bytes
+ * on this grid; 0: kernel by kernel.  One workgroup per CU, at most two tiles
+ * of FP64 cells (a thread then holds 16 cells, 128 VGPRs of r, p, A p and phi
+ * of the 256 it can have) or four of FP32 cells.  FP64 rows of more than two
+ * tiles stay with the row kernels, whose choice by row length
+ * (tests/test_gpu_rowkernel.py) the switches below describe; so does any run
+ * that sets one of those switches, times the kernels, or may not allocate. */
+static int resident_tiles(size_t esize)
+{
+  bb_resident_last = 0;
+  if (!bb_resident || cg_in_scratch || bb_time_kernels) return 0;
+  if (bb_spmv_variant != 3 || !bb_row_fp64 || bb_row_ry || bb_row_depth ||
+      !bb_row_pairs || bb_row_zc || bb_update_variant != 1 || bb_urow_fp64 ||
+      bb_urow_zc || bb_urow_depth || bb_spmv_tzb || bb_spmv_tzb32 ||
+      !bb_spmv_ntp || !bb_spmv_nts || !bb_spmv_nts32 || !bb_defer_phi ||
+      bb_pcg_batch != 16)
+    return 0;
+  if (esize == 8 && ddom.nx > 2 * TILE_X) return 0;
+  if (resident_cus == 0) {
+    int dev = 0, coop = 0;
+    BB_CHECK(hipGetDevice(&dev));
+    BB_CHECK(hipDeviceGetAttribute(&resident_cus,
+      hipDeviceAttributeMultiprocessorCount, dev));
+    BB_CHECK(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch,
+      dev));
+    if (!coop) resident_cus = -1;
+  }
+  if (resident_cus < 0) return 0;
+  const Tiles T = tiles_of(ddom);
+  if (n_tiles(ddom) > MEET_SLOTS) return 0;
+  for (int nt = 1; nt <= (esize == 8 ? 2 : 4); nt *= 2)
+    if ((long) T.ntx * T.nty * ((T.ntz + nt - 1) / nt) <= resident_cus)
+      return nt;
+  return 0;
+}
+
+template <typename V, bool MIXED, bool MASK, int NT>
+static hipError_t resident_launch(const CoefT<V> &K, const InvMT<V> &T,
+  const Sweep<V> &S)
+{
+  const Tiles G = tiles_of(ddom);
+  int ntiles = (int) n_tiles(ddom);
+  CoefT<V> k = K;
+  InvMT<V> t = T;
+  Sweep<V> s = S;
+  void *args[] = {&ddom, &k, &t, &_cg_state, &ntiles, &s};
+  return hipLaunchCooperativeKernel(
+    (const void *) resident_kernel<V, MIXED, MASK, NT>,
+    dim3((unsigned) (G.ntx * G.nty * ((G.ntz + NT - 1) / NT))),
+    dim3(TILE_THREADS), args, 0, bb_stream);
+}
+
+/* One sweep in one launch, `nt` tiles per workgroup; false: it could not be
+ * launched, and this simulation does not try again. */
+template <typename V, bool MIXED>
+static bool resident_sweep(int nt, const CoefT<V> &K, const InvMT<V> &T,
+  Sweep<V> S)
+{
+  if (!_meet)
+    BB_CHECK(hipMalloc((void **) &_meet,
+      MEET_SETS * MEET_SLOTS * sizeof(u64)));
+  S.slots = _meet;
+  S.fluid = fluid_mask();
+  S.rpart = _part_r;
+  S.spins = bb_resident_spins;
+  hipLaunchKernelGGL(meet_clear_kernel, dim3(MEET_SETS * MEET_SLOTS / 256),
+    dim3(256), 0, bb_stream, _meet);
+  hipError_t e = hipErrorInvalidValue;
+#define RS(N) e = S.fluid ? resident_launch<V, MIXED, true, N>(K, T, S) \
+                          : resident_launch<V, MIXED, false, N>(K, T, S)
+  if (nt == 1) RS(1);
+  else if (nt == 2) RS(2);
+  else if constexpr (sizeof(V) == 4) RS(4);
+#undef RS
+  if (e != hipSuccess) {
+    (void) hipGetLastError();
+    resident_cus = -1;
+    return false;
+  }
+  bb_resident_last = nt;
+  return true;
+}
+
 /* The plain FP64 Jacobi-PCG (src/cuda_solver.cu:574-761) on the RHS already
  * in _rhs_p with the tile partials of (b, b) in _part_p. */
 static void pcg_plain(double ts, int warm)
@@ -2851,18 +2956,40 @@ static void pcg_plain(double ts, int warm)
   const long nt = n_tiles(ddom);
   cg_buffers();
 
-  if (warm)
-    hipLaunchKernelGGL(cg_init_warm_kernel, TILES_LAUNCH, ddom, K, T, _rhs_p,
-      fluid_mask(), _phi, _r_q, _part_r);
-  else
-    hipLaunchKernelGGL(cg_init_kernel, TILES_LAUNCH, ddom, T, _rhs_p,
-      fluid_mask(), _r_q, _phi, _part_r);
-  hipLaunchKernelGGL(cg_state_init_kernel, dim3(1), dim3(TILE_THREADS), 0,
-    bb_stream, _part_p, _part_r, nt, _cg_state, pp_residual*pp_residual, 0.);
-  BB_LAUNCH_CHECK();
-  fetch_state();
-  real sp_rhs = cg_host->sp_rhs;
   real RHS_TOL = 1.e-8;
+  auto start = [&]() {
+    if (warm)
+      hipLaunchKernelGGL(cg_init_warm_kernel, TILES_LAUNCH, ddom, K, T, _rhs_p,
+        fluid_mask(), _phi, _r_q, _part_r);
+    else
+      hipLaunchKernelGGL(cg_init_kernel, TILES_LAUNCH, ddom, T, _rhs_p,
+        fluid_mask(), _r_q, _phi, _part_r);
+    hipLaunchKernelGGL(cg_state_init_kernel, dim3(1), dim3(TILE_THREADS), 0,
+      bb_stream, _part_p, _part_r, nt, _cg_state, pp_residual*pp_residual, 0.);
+    BB_LAUNCH_CHECK();
+  };
+  start();
+  bool one_launch = false;
+  if (int ntw = resident_tiles(sizeof(double))) {
+    Sweep<double> S = {};
+    S.r = _r_q;
+    S.phi = _phi;
+    S.pa = _p_q;
+    S.pb = _p_alt;
+    S.rhs = _rhs_p;
+    S.first = 1;
+    S.qmax = pp_max_iter + 1;
+    S.rhs_min = RHS_TOL*RHS_TOL;
+    one_launch = resident_sweep<double, false>(ntw, K, T, S);
+  }
+  fetch_state();
+  if (one_launch && cg_host->lost) {
+    resident_cus = -1;
+    one_launch = false;
+    start();
+    fetch_state();
+  }
+  real sp_rhs = cg_host->sp_rhs;
 
   pp_last.sp_rhs = sp_rhs;
   pp_last.nouter = 1;
@@ -2877,8 +3004,8 @@ static void pcg_plain(double ts, int warm)
     log_solve(0);
     return;
   }
-  int q = 0;
-  while (q <= pp_max_iter) {
+  int q = one_launch ? cg_host->q : 0;
+  while (!one_launch && q <= pp_max_iter) {
     int qend = q + (q == 0 ? first_batch(0, 0) : bb_pcg_batch);
     if (qend > pp_max_iter + 1) qend = pp_max_iter + 1;
     for (int qq = q + 1; qq <= qend; qq++) enqueue_iteration(qq, K, T);
@@ -2890,7 +3017,8 @@ static void pcg_plain(double ts, int warm)
   }
   if (cg_host->done) record_sweep(0, 0, cg_host->q);
   /* a solve that stops right after a PHI_SKIP update: add its term */
-  if (cg_host->done && cg_host->q >= 1 && phi_skips(cg_host->q)) {
+  if (!one_launch && cg_host->done && cg_host->q >= 1 &&
+      phi_skips(cg_host->q)) {
     hipLaunchKernelGGL(phi_finish_kernel<double>, TILES_LAUNCH, ddom,
       _cg_state, (cg_host->q & 1) ? _p_q : _p_alt, _phi);
     BB_LAUNCH_CHECK();
@@ -3117,18 +3245,21 @@ static void pcg_mixed(double ts, int warm)
   cg_buffers();
   cg_buffers32();
 
-  if (warm) {
-    hipLaunchKernelGGL(mx_zero_kernel, TILES_LAUNCH, ddom, _e32);
-    hipLaunchKernelGGL(mx_residual_kernel, TILES_LAUNCH, ddom, K, T, _phi,
-      _rhs_p, fluid_mask(), _r32, _part_r);
-  } else {
-    hipLaunchKernelGGL(mx_init_kernel, TILES_LAUNCH, ddom, T, _rhs_p,
-      fluid_mask(), _phi, _e32, _r32, _part_r);
-  }
-  hipLaunchKernelGGL(cg_state_init_kernel, dim3(1), dim3(TILE_THREADS), 0,
-    bb_stream, _part_p, _part_r, nt, _cg_state, pp_residual*pp_residual,
-    pp_inner_tol*pp_inner_tol);
-  BB_LAUNCH_CHECK();
+  auto start = [&](int from_phi) {
+    if (from_phi) {
+      hipLaunchKernelGGL(mx_zero_kernel, TILES_LAUNCH, ddom, _e32);
+      hipLaunchKernelGGL(mx_residual_kernel, TILES_LAUNCH, ddom, K, T, _phi,
+        _rhs_p, fluid_mask(), _r32, _part_r);
+    } else {
+      hipLaunchKernelGGL(mx_init_kernel, TILES_LAUNCH, ddom, T, _rhs_p,
+        fluid_mask(), _phi, _e32, _r32, _part_r);
+    }
+    hipLaunchKernelGGL(cg_state_init_kernel, dim3(1), dim3(TILE_THREADS), 0,
+      bb_stream, _part_p, _part_r, nt, _cg_state, pp_residual*pp_residual,
+      pp_inner_tol*pp_inner_tol);
+    BB_LAUNCH_CHECK();
+  };
+  start(warm);
   fetch_state();
   real sp_rhs = cg_host->sp_rhs;
   real RHS_TOL = 1.e-8;
@@ -3149,7 +3280,53 @@ static void pcg_mixed(double ts, int warm)
   pair_base32 = 1;
   int done = cg_host->rz1 <= pp_residual*pp_residual*sp_rhs;
   int sweep0 = 0;                       /* q at the start of the sweep */
+  /* the FP64 correction after the sweep that ended with iteration `at`, and
+   * the state it leaves */
+  auto correct = [&](int at) {
+    hipLaunchKernelGGL(mx_fold_kernel, TILES_LAUNCH, ddom, _phi, _e32);
+    hipLaunchKernelGGL(mx_residual_kernel, TILES_LAUNCH, ddom, K, T, _phi,
+      _rhs_p, fluid_mask(), _r32, _part_r);
+    hipLaunchKernelGGL(mx_state_kernel, dim3(1), dim3(TILE_THREADS), 0,
+      bb_stream, _cg_state, _part_r, nt, at, bb_mixed_restart);
+    BB_LAUNCH_CHECK();
+    fetch_state();
+  };
+  int ntw = resident_tiles(sizeof(float));
   while (!done && q <= pp_max_iter && nouter <= pp_max_iter) {
+    if (ntw) {
+      /* a sweep, its correction and the stopping test; one host read */
+      Sweep<float> S = {};
+      S.r = _r32;
+      S.phi = _e32;
+      S.pa = _p32a;
+      S.pb = _p32b;
+      S.q0 = q;
+      S.first = q + 1 == first_q;
+      S.qmax = pp_max_iter + 1;
+      if (!resident_sweep<float, true>(ntw, K32, T32, S)) {
+        ntw = 0;
+        continue;
+      }
+      correct(-1);
+      if (cg_host->lost) {
+        /* kernel by kernel from the phi of the last correction */
+        resident_cus = -1;
+        ntw = 0;
+        start(1);
+        fetch_state();
+        done = cg_host->rz1 <= pp_residual*pp_residual*sp_rhs;
+        q = sweep0 = 0;
+        first_q = pair_base32 = 1;
+        continue;
+      }
+      record_sweep(1, nouter - 1, cg_host->q - q);
+      q = sweep0 = cg_host->q;
+      pair_base32 = q + 1;
+      nouter++;
+      done = cg_host->done;
+      if (bb_mixed_restart) first_q = q + 1;
+      continue;
+    }
     int qend = q + (q == sweep0 ? first_batch(1, nouter - 1) : bb_pcg_batch);
     if (qend > pp_max_iter + 1) qend = pp_max_iter + 1;
     for (int qq = q + 1; qq <= qend; qq++)
@@ -3169,14 +3346,8 @@ static void pcg_mixed(double ts, int warm)
       hipLaunchKernelGGL(phi_finish_kernel<float>, TILES_LAUNCH, ddom,
         _cg_state, (q & 1) ? _p32a : _p32b, _e32);
     pair_base32 = q + 1;
-    hipLaunchKernelGGL(mx_fold_kernel, TILES_LAUNCH, ddom, _phi, _e32);
-    hipLaunchKernelGGL(mx_residual_kernel, TILES_LAUNCH, ddom, K, T, _phi,
-      _rhs_p, fluid_mask(), _r32, _part_r);
-    hipLaunchKernelGGL(mx_state_kernel, dim3(1), dim3(TILE_THREADS), 0,
-      bb_stream, _cg_state, _part_r, nt, q, bb_mixed_restart);
-    BB_LAUNCH_CHECK();
     nouter++;
-    fetch_state();
+    correct(q);
     done = cg_host->done;
     if (bb_mixed_restart) first_q = q + 1;
   }
