@@ -260,25 +260,20 @@ conv_fwd_kernel(TV X, int cin, int cin_pad, const uint16_t *__restrict__ W,
   }
 }
 
-/* Four consecutive channels of one voxel as loaded by the staging loop
- * of conv_lds_kernel: BF16 inputs stay packed (two registers), FP32 inputs
- * are converted to BF16 when they are written to LDS. */
+/* UC consecutive channels of one voxel (16 bytes) as loaded by the staging
+ * loop of conv_lds_kernel, and as the BF16 values it stores in LDS. */
 template <typename IN> struct RawUnit;
 template <> struct RawUnit<uint16_t> {
-  typedef u16x4 T;
-  __device__ static T zero() { return (T) 0; }
-  __device__ static void set(T &r, int e, uint16_t x) { r[e] = x; }
-  __device__ static u16x4 bf16(const T &r) { return r; }
+  typedef u16x8 T;
+  typedef u16x8 H;
+  static constexpr int UC = 8;
+  __device__ static H bf16(const T &r) { return r; }
 };
 template <> struct RawUnit<float> {
   typedef float4 T;
-  __device__ static T zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
-  __device__ static void set(T &r, int e, float x)
-  {
-    if (e == 0) r.x = x; else if (e == 1) r.y = x; else if (e == 2) r.z = x;
-    else r.w = x;
-  }
-  __device__ static u16x4 bf16(const T &r)
+  typedef u16x4 H;
+  static constexpr int UC = 4;
+  __device__ static H bf16(const T &r)
   {
     u16x4 h;
     h[0] = f2bf(r.x); h[1] = f2bf(r.y); h[2] = f2bf(r.z); h[3] = f2bf(r.w);
@@ -293,7 +288,25 @@ template <> struct RawUnit<float> {
  * in LDS, then runs the 27 taps from LDS, so each input element is read
  * from memory about 1.7 times per chunk instead of once per tap.  Output
  * channels: NCO tiles of 16 per wavefront, Cout_pad / (16 NCO) workgroups
- * along grid.y.  Same fragment layouts as conv_fwd_kernel. */
+ * along grid.y.  Same fragment layouts as conv_fwd_kernel.
+ *
+ * Every product is 16 x 16 x 32.  A chunk of 32 channels is one tap's K; a
+ * chunk of 16 (Cin_pad not a multiple of 32) takes two taps: lanes 0-31 hold
+ * the 16 channels of the first, lanes 32-63 those of the second (zero weights
+ * in the place of a 28th).
+ *
+ * No load stands behind a branch: a unit outside the volume reads voxel 0 and
+ * is replaced by zeros on its way to LDS.  Behind a branch the compiler waits
+ * for each load before the next, and the workgroup pays the latency of memory
+ * once per unit (the kernel before: 11 units of 8 bytes, 16 x 16 x 16
+ * products for 16 channels).  At 128^3: 16 channels 179 us before, 100 now;
+ * 32 channels 68 and 64, now 55 and 51; the forward pass 1199 us before, 831
+ * now.  The staging's latency still bounds the 16-channel layers, whose
+ * products take a sixth of the time.  Needs cin = Cin_pad and rows that are aligned to
+ * the 16-byte units.
+ *
+ * M.p: the output (FP32) is zeroed where the BF16 tensor M is not positive,
+ * the ReLU of the layer whose output gradient this is. */
 #define CB_X 16
 #define CB_Y 4
 #define CB_Z 4
@@ -301,115 +314,123 @@ template <> struct RawUnit<float> {
 
 template <typename IN, int KS, int NCO>
 __global__ void __launch_bounds__(256)
-conv_lds_kernel(TV X, int cin, int cin_pad, const uint16_t *__restrict__ W,
+conv_lds_kernel(TV X, int cin_pad, const uint16_t *__restrict__ W,
   const float *__restrict__ bias, int cout, int cout_pad, TV Yf, TV Yb,
-  int relu, int vec)
+  int relu, TV M)
 {
-  constexpr int NT = 4, KPL = KS / 4;
-  constexpr int KCP = KS + 8;           /* LDS row: KS channels + padding */
-  /* taps per weight group: a z-plane of taps (9) where their fragments
-   * take at most 72 registers (KPL / 2 per fragment), else a row (3);
-   * all 27 at once cost the 16-channel kernel an occupancy step */
-  constexpr int TG = NCO * KPL * 9 <= 144 ? 9 : 3;
-  typedef typename Frag<KS>::T F;
-  typedef typename U16V<KPL>::T U;
+  constexpr int NT = 4;
+  constexpr int UC = RawUnit<IN>::UC;
+  /* LDS row: 16 channels pack 32-byte rows that a wavefront reads without
+   * conflicts; 32 channels are padded to 80 bytes */
+  constexpr int KCP = KS == 16 ? 16 : KS + 8;
+  constexpr int NS = KS == 16 ? 14 : 27;        /* products over the taps */
+  /* products per group of weight fragments, loaded together */
+  constexpr int TG = KS == 16 ? (NCO <= 2 ? 7 : 2) : (NCO <= 2 ? 9 : 3);
+  typedef typename RawUnit<IN>::T RU;
+  typedef typename RawUnit<IN>::H RH;
   __shared__ __attribute__((aligned(16))) uint16_t tile[CB_V * KCP];
-  int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  int q = lane >> 4, n = lane & 15;
-  int nbx = (X.nx + CB_X - 1) / CB_X, nby = (X.ny + CB_Y - 1) / CB_Y;
-  int b = blockIdx.x;
-  int x0 = (b % nbx) * CB_X, y0 = ((b / nbx) % nby) * CB_Y,
-      z0 = (b / (nbx * nby)) * CB_Z;
-  int co0 = blockIdx.y * 16 * NCO;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int q = lane >> 4, n = lane & 15;
+  const int nbx = (X.nx + CB_X - 1) / CB_X, nby = (X.ny + CB_Y - 1) / CB_Y;
+  const int b = blockIdx.x;
+  const int x0 = (b % nbx) * CB_X, y0 = ((b / nbx) % nby) * CB_Y,
+            z0 = (b / (nbx * nby)) * CB_Z;
+  const int co0 = blockIdx.y * 16 * NCO;
   f32x4 acc[NT][NCO];
 #pragma unroll
   for (int t = 0; t < NT; t++)
 #pragma unroll
     for (int c = 0; c < NCO; c++) acc[t][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const uint16_t *Wl = W + (long) (co0 + n) * cin_pad + KPL * q;
+
+  /* the units this thread stages: voxel row of X (0 where outside) */
+  constexpr int UV = KS / UC, NUNIT = CB_V * UV, NU = (NUNIT + 255) / 256;
+  unsigned row[NU], inside = 0;
+#pragma unroll
+  for (int i = 0; i < NU; i++) {
+    const int u = threadIdx.x + 256 * i, v = u / UV;
+    const int gx = x0 + v % (CB_X + 2) - 1,
+              gy = y0 + (v / (CB_X + 2)) % (CB_Y + 2) - 1,
+              gz = z0 + v / ((CB_X + 2) * (CB_Y + 2)) - 1;
+    const bool in = u < NUNIT && gx >= 0 && gy >= 0 && gz >= 0 &&
+                    gx < X.nx && gy < X.ny && gz < X.nz;
+    row[i] = in ? (unsigned) gx + (unsigned) X.nx *
+                  ((unsigned) gy + (unsigned) X.ny * (unsigned) gz) : 0u;
+    inside |= (unsigned) in << i;
+  }
+  const IN *Xc = (const IN *) X.p + X.c0 + UC * (threadIdx.x % UV);
+  const bool hi = q >= 2;
+  const int kq = KS == 16 ? 8 * (q & 1) : 8 * q;  /* this lane's channels */
+  const uint16_t *Wl = W + (long) (co0 + n) * cin_pad + kq;
+  /* first input voxel of row t of this wavefront and column n, tap (0,0,0) */
+  const int vb = KCP * (n + (CB_X + 2) * (CB_Y + 2) * wv) + kq;
+  static_assert(NT == CB_Y, "a wavefront takes the rows of one z plane");
+
   for (int ch = 0; ch < cin_pad; ch += KS) {
-    /* stage: units of 4 channels of one voxel, NU per thread.  Every load
-     * of the chunk is issued before the first LDS store, so the
-     * workgroup waits for its loads once and not once per unit. */
-    constexpr int NUNIT = CB_V * (KS / 4), NU = (NUNIT + 255) / 256;
-    /* BF16 input: the four channels packed as loaded; FP32: four floats */
-    typedef typename RawUnit<IN>::T RU;
     RU rv[NU];
 #pragma unroll
-    for (int i = 0; i < NU; i++) {
-      const int u = threadIdx.x + 256 * i;
-      rv[i] = RawUnit<IN>::zero();
-      const int v = u / (KS / 4), c4 = 4 * (u % (KS / 4));
-      const int vx = v % (CB_X + 2), vy = (v / (CB_X + 2)) % (CB_Y + 2),
-                vz = v / ((CB_X + 2) * (CB_Y + 2));
-      const int gx = x0 + vx - 1, gy = y0 + vy - 1, gz = z0 + vz - 1;
-      if (u < NUNIT && gx >= 0 && gy >= 0 && gz >= 0 && gx < X.nx &&
-          gy < X.ny && gz < X.nz) {
-        long row = (long) gx + (long) X.nx * (gy + (long) X.ny * gz);
-        int c = ch + c4;
-        const IN *p = (const IN *) X.p + row * X.ld + X.c0 + c;
-        if (vec && c + 4 <= cin) {
-          rv[i] = *(const RU *) p;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; e++)
-            if (c + e < cin) RawUnit<IN>::set(rv[i], e, p[e]);
-        }
-      }
-    }
+    for (int i = 0; i < NU; i++)
+      rv[i] = *(const RU *) (Xc + (size_t) row[i] * X.ld + ch);
+    if (ch > 0) __syncthreads();      /* the last chunk's products are done */
 #pragma unroll
     for (int i = 0; i < NU; i++) {
       const int u = threadIdx.x + 256 * i;
-      if (u < NUNIT) {
-        const int v = u / (KS / 4), c4 = 4 * (u % (KS / 4));
-        *(u16x4 *) &tile[v * KCP + c4] = RawUnit<IN>::bf16(rv[i]);
-      }
+      const RH h = (inside >> i) & 1u ? RawUnit<IN>::bf16(rv[i]) : (RH) 0;
+      if (u < NUNIT)
+        *(RH *) &tile[(u / UV) * KCP + UC * (u % UV)] = h;
     }
     __syncthreads();
-    /* taps in groups of TG: the group's weight fragments are loaded
-     * together before its MFMAs, so their latency is paid once per group
-     * and not once per tap (same MFMAs in the same order) */
-    for (int g0 = 0; g0 < 27; g0 += TG) {
-      F aw[TG][NCO];
+#pragma clang loop unroll_count(KS == 16 ? NS : 1)
+    for (int g0 = 0; g0 < NS; g0 += TG) {
+      bf16x8 aw[TG][NCO];
 #pragma unroll
-      for (int tg = 0; tg < TG; tg++)
+      for (int s = 0; s < TG; s++) {
+        if (g0 + s >= NS) continue;
+        /* a tap, or the lane's tap of two */
+        const int tap = KS == 16 ? min(2 * (g0 + s) + (hi ? 1 : 0), 26)
+                                 : g0 + s;
+        const bool none = KS == 16 && g0 + s == 13 && hi;
 #pragma unroll
-        for (int c = 0; c < NCO; c++)
-          aw[tg][c] = load_w<KS>(Wl + (long) (g0 + tg) * cout_pad * cin_pad +
-                                 ch + (long) c * 16 * cin_pad);
-#pragma unroll
-      for (int tg = 0; tg < TG; tg++) {
-        const int tap = g0 + tg;
-        int dx = tap % 3, dy = (tap / 3) % 3, dz = tap / 9;   /* offset + 1 */
-        F bfr[NT];
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-          int r = wv * NT + t;
-          int yy = r % CB_Y, zz = r / CB_Y;
-          int v = (n + dx) + (CB_X + 2) * ((yy + dy) + (CB_Y + 2) * (zz + dz));
-          bfr[t] = __builtin_bit_cast(F, *(const U *) &tile[v * KCP + KPL * q]);
+        for (int c = 0; c < NCO; c++) {
+          const bf16x8 w = load_w<32>(Wl + (long) tap * cout_pad * cin_pad +
+                                      ch + (long) c * 16 * cin_pad);
+          aw[s][c] = none ? __builtin_bit_cast(bf16x8, (u16x8) 0) : w;
         }
+      }
+#pragma unroll
+      for (int s = 0; s < TG; s++) {
+        if (g0 + s >= NS) continue;
+        auto at = [](int tap) {
+          return KCP * (tap % 3 + (CB_X + 2) * ((tap / 3) % 3 +
+                                               (CB_Y + 2) * (tap / 9)));
+        };
+        const int ta = KS == 16 ? 2 * (g0 + s) : g0 + s;
+        const int o = KS == 16 ? vb + (hi ? at(ta + 1 < 27 ? ta + 1 : 26)
+                                          : at(ta)) : vb + at(ta);
+        bf16x8 bfr[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+          bfr[t] = __builtin_bit_cast(bf16x8,
+            *(const u16x8 *) &tile[o + KCP * (CB_X + 2) * t]);
 #pragma unroll
         for (int c = 0; c < NCO; c++)
 #pragma unroll
           for (int t = 0; t < NT; t++)
-            acc[t][c] = mfma_bf16<KS>(aw[tg][c], bfr[t], acc[t][c]);
+            acc[t][c] = mfma_bf16<32>(aw[s][c], bfr[t], acc[t][c]);
       }
     }
-    __syncthreads();
   }
   /* D[m][n]: lane holds output channels co0 + 16 c + 4 q + e of voxel n of
-   * row wv * NT + t */
+   * row t of plane wv */
   const TV &O = Yf.p ? Yf : Yb;
 #pragma unroll
   for (int t = 0; t < NT; t++) {
-    int r = wv * NT + t;
-    int gx = x0 + n, gy = y0 + r % CB_Y, gz = z0 + r / CB_Y;
+    const int gx = x0 + n, gy = y0 + t, gz = z0 + wv;
     if (gx >= O.nx || gy >= O.ny || gz >= O.nz) continue;
-    long v = (long) gx + (long) O.nx * (gy + (long) O.ny * gz);
+    const long v = (long) gx + (long) O.nx * (gy + (long) O.ny * gz);
 #pragma unroll
     for (int c = 0; c < NCO; c++) {
-      int cb = co0 + 16 * c + 4 * q;
+      const int cb = co0 + 16 * c + 4 * q;
       if (cb >= cout) continue;
       float val[4];
 #pragma unroll
@@ -417,6 +438,12 @@ conv_lds_kernel(TV X, int cin, int cin_pad, const uint16_t *__restrict__ W,
         float bb = (bias && cb + e < cout) ? bias[cb + e] : 0.f;
         val[e] = acc[t][c][e] + bb;
         if (relu) val[e] = val[e] > 0.f ? val[e] : 0.f;
+      }
+      if (M.p) {
+        const uint16_t *m = (const uint16_t *) M.p + v * M.ld + M.c0 + cb;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (cb + e < cout && !(bf2f(m[e]) > 0.f)) val[e] = 0.f;
       }
       bool full = cb + 4 <= cout && (O.ld & 3) == 0 && (O.c0 & 3) == 0;
       if (Yf.p) {
@@ -439,78 +466,221 @@ conv_lds_kernel(TV X, int cin, int cin_pad, const uint16_t *__restrict__ W,
   }
 }
 
-/* Weight gradient partials: P[chunk][tap][co][ci] = sum over the chunk's
- * voxels v of G[v, co] X[v + off(tap), ci].  Grid: (nchunks, taps *
- * cout_pad/16 * cin_pad/16 / 4); 4 wavefronts, each one (tap, co-tile,
- * ci-tile).  G is FP32, X is BF16. */
-__global__ void __launch_bounds__(256)
-conv_wgrad_kernel(TV G, int cout, TV X, int cin, int taps, int cout_pad,
-  int cin_pad, long chunk, float *__restrict__ P)
+/* Weight- and bias-gradient partials of a chunk of voxels:
+ * P[chunk][tap][co][ci] = sum of G[v, co] X[v + off(tap), ci] and
+ * Pb[chunk][co] = sum of G[v, co] over the chunk's voxels (G FP32, X BF16).
+ *
+ * A workgroup takes one chunk, 16 input channels (blockIdx.y) and every tap
+ * and output channel.  Blocks of 16 x 4 x 4 voxels of G (rounded to BF16) and
+ * of the 18 x 6 x 6 voxels of X around them pass through LDS as they lie in
+ * memory, 16 channels to a voxel; the products' K index is the voxel, so both
+ * operands are read transposed: ds_read_b64_tr_b16 gives lane i of each group
+ * of 16 lanes channel i of four voxels.  A row of 16 voxels is then 512
+ * consecutive bytes for the wavefront whatever the tap, free of bank
+ * conflicts, and a tap is a constant added to the address.  Taps are shared
+ * out over the four wavefronts (TAPS = 1: the voxels are).  X has Cin_pad
+ * channels (zeros past the layer's own) in rows aligned to 16 bytes.
+ *
+ * The kernel that this replaces gathered every operand element by itself from
+ * memory, 16 voxels per product, once per tap, and summed the bias in a pass
+ * of one thread per channel: 219 and 51 us per layer (mean over the eleven
+ * layers of a 64^3 crop) where this one takes 13 to 21.  What bounds it now is
+ * the 18 x 6 x 6 staging (2.5 times the voxels of a block) behind one barrier
+ * per block; four training steps of that crop went from 20.6 to 4.2 ms. */
+__device__ inline u16x4 lds_read_tr(const uint16_t *p)
 {
-  int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  int nco = cout_pad / 16, nci = cin_pad / 16;
-  int job = blockIdx.y * 4 + wv;
-  if (job >= taps * nco * nci) return;
-  int tap = job / (nco * nci), rem = job % (nco * nci);
-  int co0 = (rem / nci) * 16, ci0 = (rem % nci) * 16;
-  int dx = 0, dy = 0, dz = 0;
-  if (taps == 27) { dx = tap % 3 - 1; dy = (tap / 3) % 3 - 1; dz = tap / 9 - 1; }
-  long nv = (long) G.nx * G.ny * G.nz;
-  long vb = (long) blockIdx.x * chunk, ve = vb + chunk < nv ? vb + chunk : nv;
-  int m = lane & 15, kq = 4 * (lane >> 4);
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (long v0 = vb; v0 < ve; v0 += 16) {
-    bf16x4 a = {0, 0, 0, 0}, b = {0, 0, 0, 0};
-    for (int e = 0; e < 4; e++) {
-      long v = v0 + kq + e;
-      int x, y, z;
-      if (v >= ve || !vox_xyz(G, v, &x, &y, &z)) continue;
-      if (co0 + m < cout)
-        a[e] = (short) f2bf(((const float *) G.p)[v * G.ld + G.c0 + co0 + m]);
-      int xs = x + dx, ys = y + dy, zs = z + dz;
-      if (ci0 + m < cin && xs >= 0 && ys >= 0 && zs >= 0 && xs < X.nx &&
-          ys < X.ny && zs < X.nz) {
-        long vs = (long) xs + (long) X.nx * (ys + (long) X.ny * zs);
-        b[e] = (short) ((const uint16_t *) X.p)[vs * X.ld + X.c0 + ci0 + m];
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4 *LP;
+  return __builtin_bit_cast(u16x4,
+    __builtin_amdgcn_ds_read_tr16_b64_v4i16((LP) p));
+}
+
+/* A or B operand of a 16x16x32 product: the 16 channels of the 2 x 16 voxels
+ * at p and p + 2nd, transposed. */
+__device__ inline bf16x8 lds_frag_tr(const uint16_t *p, int second)
+{
+  const u16x4 a = lds_read_tr(p), b = lds_read_tr(p + second);
+  u16x8 r;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    r[e] = a[e];
+    r[e + 4] = b[e];
+  }
+  return __builtin_bit_cast(bf16x8, r);
+}
+
+template <int TAPS, int NCO>
+__global__ void __launch_bounds__(256)
+wgrad_kernel(TV G, int cout, TV X, int cin_pad, int nblocks,
+  float *__restrict__ P, float *__restrict__ Pb)
+{
+  constexpr int TW = TAPS == 27 ? 7 : 1;         /* taps per wavefront */
+  constexpr int UG = 4 * NCO;                    /* float4 units per voxel */
+  constexpr int NX = TAPS == 27 ? CB_V : 256;    /* voxels of X in LDS */
+  __shared__ __attribute__((aligned(16))) uint16_t s_x[NX * 16];
+  __shared__ __attribute__((aligned(16))) uint16_t s_g[NCO][256 * 16];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int nbx = (G.nx + CB_X - 1) / CB_X, nby = (G.ny + CB_Y - 1) / CB_Y;
+  const int c0 = blockIdx.y * 16;
+  f32x4 acc[TW][NCO];
+  int tapoff[TW];
+#pragma unroll
+  for (int i = 0; i < TW; i++) {
+    const int tap = min(wv * TW + i, TAPS - 1);
+    tapoff[i] = TAPS == 27 ? 16 * (tap % 3 + (CB_X + 2) * ((tap / 3) % 3 +
+                                              (CB_Y + 2) * (tap / 9))) : 0;
+#pragma unroll
+    for (int c = 0; c < NCO; c++) acc[i][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  }
+  float4 bsum = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int cg = 4 * (t % UG);                   /* this thread's channels of G */
+  const bool vecg = G.ld % 4 == 0 && G.c0 % 4 == 0 && cout == 16 * NCO;
+
+  for (int b = blockIdx.x; b < nblocks; b += gridDim.x) {
+    const int x0 = (b % nbx) * CB_X, y0 = ((b / nbx) % nby) * CB_Y,
+              z0 = (b / (nbx * nby)) * CB_Z;
+    /* G: voxels t / UG + 256 / UG i, four channels each; X: units of eight
+     * channels, the voxels around included.  Loads without a branch (voxel 0
+     * where there is none, zeros instead on the way to LDS), as in
+     * conv_lds_kernel: all are in flight together. */
+    float4 g[UG];
+    unsigned gin = 0, xin = 0;
+#pragma unroll
+    for (int i = 0; i < UG; i++) {
+      const int v = t / UG + (256 / UG) * i;
+      const int gx = x0 + v % CB_X, gy = y0 + (v / CB_X) % CB_Y,
+                gz = z0 + v / (CB_X * CB_Y);
+      const bool in = gx < G.nx && gy < G.ny && gz < G.nz;
+      const unsigned row = in ? (unsigned) gx + (unsigned) G.nx *
+                           ((unsigned) gy + (unsigned) G.ny * (unsigned) gz) : 0u;
+      gin |= (unsigned) in << i;
+      const float *p = (const float *) G.p + (size_t) row * G.ld + G.c0;
+      if (vecg) {
+        g[i] = *(const float4 *) (p + cg);
+      } else {
+        const int last = cout - 1;
+        const float a = p[min(cg, last)], b1 = p[min(cg + 1, last)],
+                    c = p[min(cg + 2, last)], d = p[min(cg + 3, last)];
+        g[i] = make_float4(cg <= last ? a : 0.f, cg + 1 <= last ? b1 : 0.f,
+                           cg + 2 <= last ? c : 0.f, cg + 3 <= last ? d : 0.f);
       }
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+    constexpr int NU = (2 * NX + 255) / 256;
+    u16x8 xv[NU];
+#pragma unroll
+    for (int i = 0; i < NU; i++) {
+      const int u = t + 256 * i, v = u >> 1;
+      constexpr int W = TAPS == 27 ? CB_X + 2 : CB_X,
+                    H = TAPS == 27 ? CB_Y + 2 : CB_Y, O = TAPS == 27 ? 1 : 0;
+      const int gx = x0 + v % W - O, gy = y0 + (v / W) % H - O,
+                gz = z0 + v / (W * H) - O;
+      const bool in = u < 2 * NX && gx >= 0 && gy >= 0 && gz >= 0 &&
+                      gx < X.nx && gy < X.ny && gz < X.nz;
+      const unsigned row = in ? (unsigned) gx + (unsigned) X.nx *
+                           ((unsigned) gy + (unsigned) X.ny * (unsigned) gz) : 0u;
+      xin |= (unsigned) in << i;
+      xv[i] = *(const u16x8 *) ((const uint16_t *) X.p + (size_t) row * X.ld +
+                                X.c0 + c0 + 8 * (u & 1));
+    }
+    __syncthreads();                 /* the last block's products are done */
+#pragma unroll
+    for (int i = 0; i < UG; i++) {
+      const int v = t / UG + (256 / UG) * i;
+      u16x4 h;
+      if (!((gin >> i) & 1u)) g[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      h[0] = f2bf(g[i].x); h[1] = f2bf(g[i].y);
+      h[2] = f2bf(g[i].z); h[3] = f2bf(g[i].w);
+      *(u16x4 *) &s_g[cg / 16][v * 16 + cg % 16] = h;
+      bsum.x += g[i].x; bsum.y += g[i].y; bsum.z += g[i].z; bsum.w += g[i].w;
+    }
+#pragma unroll
+    for (int i = 0; i < NU; i++) {
+      const int u = t + 256 * i;
+      if (u < 2 * NX)
+        *(u16x8 *) &s_x[(u >> 1) * 16 + 8 * (u & 1)] =
+          (xin >> i) & 1u ? xv[i] : (u16x8) 0;
+    }
+    __syncthreads();
+    /* 32 voxels (two rows along x) per product; voxel 4 (lane / 16) + j of a
+     * row, channels 4 (lane % 4) .., is at byte 8 lane of the row */
+    for (int k = TAPS == 27 ? 0 : wv; k < 8; k += TAPS == 27 ? 1 : 4) {
+      bf16x8 a[NCO];
+#pragma unroll
+      for (int c = 0; c < NCO; c++)
+        a[c] = lds_frag_tr(&s_g[c][2 * k * 256 + 4 * lane], 256);
+      /* rows 2k and 2k + 1: y = 2 (k % 2), z = k / 2 */
+      const int r = TAPS == 27 ? 16 * (CB_X + 2) * (2 * (k & 1) +
+                                   (CB_Y + 2) * (k >> 1)) : 2 * k * 256;
+      const int next = TAPS == 27 ? 16 * (CB_X + 2) : 256;
+#pragma unroll
+      for (int i = 0; i < TW; i++) {
+        const bf16x8 x = lds_frag_tr(&s_x[r + tapoff[i] + 4 * lane], next);
+#pragma unroll
+        for (int c = 0; c < NCO; c++)
+          acc[i][c] = mfma_bf16<32>(a[c], x, acc[i][c]);
+      }
+    }
   }
-  /* D[m = co][n = ci] */
-  int nn = lane & 15;
-  float *Pc = P + (long) blockIdx.x * taps * cout_pad * cin_pad;
-  for (int e = 0; e < 4; e++) {
-    int co = co0 + 4 * (lane >> 4) + e;
-    Pc[((long) tap * cout_pad + co) * cin_pad + ci0 + nn] = acc[e];
+
+  /* D[m = co][n = ci]; TAPS = 1: each wavefront is a chunk of its own */
+  const int coutp = 16 * NCO;
+  const long chunk = TAPS == 27 ? blockIdx.x : 4 * blockIdx.x + wv;
+  float *Pc = P + chunk * TAPS * coutp * cin_pad;
+#pragma unroll
+  for (int i = 0; i < TW; i++) {
+    const int tap = TAPS == 27 ? wv * TW + i : 0;
+    if (tap >= TAPS) continue;
+#pragma unroll
+    for (int c = 0; c < NCO; c++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int co = 16 * c + 4 * (lane >> 4) + e;
+        Pc[((long) tap * coutp + co) * cin_pad + c0 + (lane & 15)] = acc[i][c][e];
+      }
+  }
+  if (blockIdx.y != 0) return;
+  /* bias: the threads of one channel group, in thread order */
+  __syncthreads();
+  float4 *s_b = (float4 *) &s_g[0][0];
+  s_b[t] = bsum;
+  __syncthreads();
+  if (t < UG) {
+    float4 s = s_b[t];
+    for (int i = t + UG; i < 256; i += UG) {
+      s.x += s_b[i].x; s.y += s_b[i].y; s.z += s_b[i].z; s.w += s_b[i].w;
+    }
+    *(float4 *) &Pb[(long) blockIdx.x * coutp + 4 * t] = s;
   }
 }
 
-/* dW = sum of the chunk partials in chunk order; db[co] likewise from the
- * bias partials. */
-__global__ void sum_chunks_kernel(const float *__restrict__ P, long n,
-  int nchunks, float *__restrict__ out)
+/* gw and gb: the sums of the partials over their chunks, 32 elements and
+ * eight runs of chunks per workgroup (each run in chunk order, then the
+ * runs).  One thread per element, all chunks in turn, took 55 us per layer;
+ * this takes 8 where the partials take 1 to 5 to read. */
+__global__ void __launch_bounds__(256)
+sum_chunks_kernel(const float *__restrict__ P, long n, int nchunks,
+  float *__restrict__ gw, const float *__restrict__ Pb, int nb, int nchunksb,
+  float *__restrict__ gb)
 {
-  long i = (long) blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float s = 0.f;
-  for (int c = 0; c < nchunks; c++) s += P[(long) c * n + i];
-  out[i] = s;
-}
-
-/* Bias-gradient partials: Pb[chunk][co] = sum over the chunk of G[v, co];
- * zero for the padding channels co >= cout. */
-__global__ void bias_grad_kernel(TV G, int cout, long chunk, float *Pb)
-{
-  int co = threadIdx.x;
-  if (co >= cout) {
-    Pb[(long) blockIdx.x * blockDim.x + co] = 0.f;
-    return;
-  }
-  long nv = (long) G.nx * G.ny * G.nz;
-  long vb = (long) blockIdx.x * chunk, ve = vb + chunk < nv ? vb + chunk : nv;
-  float s = 0.f;
-  for (long v = vb; v < ve; v++) s += ((const float *) G.p)[v * G.ld + G.c0 + co];
-  Pb[(long) blockIdx.x * blockDim.x + co] = s;
+  __shared__ float s[8][32];
+  const int e = threadIdx.x & 31, r = threadIdx.x >> 5;
+  const long nwg = (n + 31) / 32;
+  const bool bias = blockIdx.x >= nwg;
+  const float *src = bias ? Pb : P;
+  const long m = bias ? nb : n;
+  const int nc = bias ? nchunksb : nchunks;
+  const long i = (bias ? blockIdx.x - nwg : blockIdx.x) * 32L + e;
+  float a = 0.f;
+  if (i < m)
+#pragma unroll 4
+    for (int c = r; c < nc; c += 8) a += src[(long) c * m + i];
+  s[r][e] = a;
+  __syncthreads();
+  if (r != 0 || i >= m) return;
+#pragma unroll
+  for (int q = 1; q < 8; q++) a += s[q][e];
+  (bias ? gb : gw)[i] = a;
 }
 
 /* Backward-data weights: Wt[tap][ci][co] = W[26 - tap][co][ci] (flipped,
@@ -795,15 +965,14 @@ static void free_acts(Acts &A)
   memset(&A, 0, sizeof(A));
 }
 
-/* Voxel chunk of the weight- and bias-gradient partials: at most
- * MAX_CHUNKS chunks of at least 256 voxels (a multiple of 16), so that a
- * 64^3 training crop spreads over 512 workgroups per tile job. */
-#define MAX_CHUNKS 512L
-static long chunk_of(long nv)
+/* Chunks of the weight-gradient partials (workgroups per 16 input channels):
+ * two or three workgroups per CU over the input channels, and no more chunks
+ * than blocks of voxels. */
+#define WGRAD_WGS 640
+static int wgrad_chunks(int nblocks, int nci)
 {
-  long c = (nv + MAX_CHUNKS - 1) / MAX_CHUNKS;
-  c = c < 256 ? 256 : c;
-  return (c + 15) / 16 * 16;
+  const int c = WGRAD_WGS / nci;
+  return c < nblocks ? c : nblocks;
 }
 
 /* Activation buffers for a volume nx x ny x nz (each divisible by 4). */
@@ -859,7 +1028,17 @@ extern "C" int bb_unet_volume(int nx, int ny, int nz)
   A.g_d0 = (float *) dzalloc(n0 * 16 * 4);
   A.g_y = (float *) dzalloc(n0 * 4);
   A.g_in0 = (float *) dzalloc(n0 * 16 * 4);
-  A.part_n = MAX_CHUNKS * 27L * 64 * 96;
+  /* partials of the layer that needs most, weights and bias */
+  A.part_n = 0;
+  for (int l = 0; l < NLAYER; l++) {
+    const Layer &Y = net->L[l];
+    const int *d = A.n[Y.level];
+    const long c = (Y.taps == 27 ? 1 : 4) * wgrad_chunks(
+      ((d[0] + CB_X - 1) / CB_X) * ((d[1] + CB_Y - 1) / CB_Y) *
+      ((d[2] + CB_Z - 1) / CB_Z), Y.cinp / 16);
+    const long need = c * (Y.nw + Y.coutp);
+    A.part_n = need > A.part_n ? need : A.part_n;
+  }
   A.part = (float *) dzalloc(A.part_n * 4);
   A.loss_n = blocks(n0, 256);
   A.loss_part = (float *) dzalloc(A.loss_n * 4);
@@ -882,6 +1061,18 @@ static TV none(void)
   return T;
 }
 
+template <typename K, typename... Args>
+static void ew(K kern, long n, Args... args)
+{
+  hipLaunchKernelGGL(kern, dim3(blocks(n, 256)), dim3(256), 0, bb_stream,
+    args...);
+}
+
+static void relu_bwd(TV G, TV Y, int C)
+{
+  ew(relu_bwd_kernel, (long) G.nx * G.ny * G.nz * C, G, Y, C);
+}
+
 /* Launch of conv_fwd_kernel: K step 32 where the input channels allow,
  * up to four output-channel tiles per wavefront. */
 int bb_unet_conv_lds = 1;    /* 3x3x3 convolutions: 1 LDS-staged kernel,
@@ -889,20 +1080,21 @@ int bb_unet_conv_lds = 1;    /* 3x3x3 convolutions: 1 LDS-staged kernel,
 
 template <typename IN>
 static void conv_launch(TV X, int cin, int cinp, const uint16_t *W, int taps,
-  const float *bias, int cout, int coutp, TV Yf, TV Yb, int relu)
+  const float *bias, int cout, int coutp, TV Yf, TV Yb, int relu,
+  TV M = none())
 {
   int ks = cinp % 32 == 0 ? 32 : 16, kpl = ks / 4;
   int tiles = coutp / 16;
   int nco = tiles % 4 == 0 ? 4 : (tiles % 3 == 0 ? 3 : (tiles % 2 == 0 ? 2 : 1));
   long nv = (long) X.nx * X.ny * X.nz;
-  if (taps == 27 && bb_unet_conv_lds) {
-    int vec4 = X.ld % 4 == 0 && X.c0 % 4 == 0;
+  const int uc = RawUnit<IN>::UC;
+  if (taps == 27 && bb_unet_conv_lds && cin == cinp && X.ld % uc == 0 &&
+      X.c0 % uc == 0) {
     long nb = (long) ((X.nx + CB_X - 1) / CB_X) * ((X.ny + CB_Y - 1) / CB_Y) *
               ((X.nz + CB_Z - 1) / CB_Z);
     dim3 g((unsigned) nb, tiles / nco);
 #define CONV_S(KS, NCO) hipLaunchKernelGGL((conv_lds_kernel<IN, KS, NCO>), \
-    g, dim3(256), 0, bb_stream, X, cin, cinp, W, bias, cout, coutp, Yf, Yb, \
-    relu, vec4)
+    g, dim3(256), 0, bb_stream, X, cinp, W, bias, cout, coutp, Yf, Yb, relu, M)
     if (ks == 32) {
       if (nco == 4) CONV_S(32, 4);
       else if (nco == 3) CONV_S(32, 3);
@@ -935,25 +1127,18 @@ static void conv_launch(TV X, int cin, int cinp, const uint16_t *W, int taps,
     else CONV_L(16, 1);
   }
 #undef CONV_L
+  if (M.p) relu_bwd(Yf, M, cout);
   BB_LAUNCH_CHECK();
 }
 
-static void conv(int l, TV X, bool xf32, TV Yf, TV Yb)
+static void conv(int l, TV X, TV Yf, TV Yb)
 {
   Layer &Y = net->L[l];
-  if (xf32)
-    conv_launch<float>(X, Y.cin, Y.cinp, Y.wb, Y.taps, Y.b, Y.cout, Y.coutp,
-                       Yf, Yb, Y.relu);
-  else
-    conv_launch<uint16_t>(X, Y.cin, Y.cinp, Y.wb, Y.taps, Y.b, Y.cout,
-                          Y.coutp, Yf, Yb, Y.relu);
-}
-
-template <typename K, typename... Args>
-static void ew(K kern, long n, Args... args)
-{
-  hipLaunchKernelGGL(kern, dim3(blocks(n, 256)), dim3(256), 0, bb_stream,
-    args...);
+  /* the input's rows hold zeros in the channels past the first layer's two,
+   * as its weights do */
+  const int cin = l == 0 ? Y.cinp : Y.cin;
+  conv_launch<uint16_t>(X, cin, Y.cinp, Y.wb, Y.taps, Y.b, Y.cout, Y.coutp,
+                        Yf, Yb, Y.relu);
 }
 
 /* Launch of a kernel with one thread per four channels of each of nv
@@ -975,57 +1160,58 @@ static void vox4(K kern, long nv, int C, Args... args)
 static void forward(void)
 {
   Acts &A = *net->A;
-  conv(0, tv(A.in0, 16, 0, A, 0), false, none(), tv(A.e0a, 16, 0, A, 0));
-  conv(1, tv(A.e0a, 16, 0, A, 0), false, none(), tv(A.cat0, 48, 32, A, 0));
+  conv(0, tv(A.in0, 16, 0, A, 0), none(), tv(A.e0a, 16, 0, A, 0));
+  conv(1, tv(A.e0a, 16, 0, A, 0), none(), tv(A.cat0, 48, 32, A, 0));
   vox4(pool_fwd_kernel, A.nv[1], 16, tv(A.cat0, 48, 32, A, 0),
        tv(A.p0, 16, 0, A, 1), 16);
-  conv(2, tv(A.p0, 16, 0, A, 1), false, none(), tv(A.e1a, 32, 0, A, 1));
-  conv(3, tv(A.e1a, 32, 0, A, 1), false, none(), tv(A.cat1, 96, 64, A, 1));
+  conv(2, tv(A.p0, 16, 0, A, 1), none(), tv(A.e1a, 32, 0, A, 1));
+  conv(3, tv(A.e1a, 32, 0, A, 1), none(), tv(A.cat1, 96, 64, A, 1));
   vox4(pool_fwd_kernel, A.nv[2], 32, tv(A.cat1, 96, 64, A, 1),
        tv(A.p1, 32, 0, A, 2), 32);
-  conv(4, tv(A.p1, 32, 0, A, 2), false, none(), tv(A.b0, 64, 0, A, 2));
-  conv(5, tv(A.b0, 64, 0, A, 2), false, none(), tv(A.b1, 64, 0, A, 2));
+  conv(4, tv(A.p1, 32, 0, A, 2), none(), tv(A.b0, 64, 0, A, 2));
+  conv(5, tv(A.b0, 64, 0, A, 2), none(), tv(A.b1, 64, 0, A, 2));
   vox4(up_fwd_kernel, A.nv[1], 64, tv(A.b1, 64, 0, A, 2),
        tv(A.cat1, 96, 0, A, 1), 64);
-  conv(6, tv(A.cat1, 96, 0, A, 1), false, none(), tv(A.d1a, 32, 0, A, 1));
-  conv(7, tv(A.d1a, 32, 0, A, 1), false, none(), tv(A.d1, 32, 0, A, 1));
+  conv(6, tv(A.cat1, 96, 0, A, 1), none(), tv(A.d1a, 32, 0, A, 1));
+  conv(7, tv(A.d1a, 32, 0, A, 1), none(), tv(A.d1, 32, 0, A, 1));
   vox4(up_fwd_kernel, A.nv[0], 32, tv(A.d1, 32, 0, A, 1),
        tv(A.cat0, 48, 0, A, 0), 32);
-  conv(8, tv(A.cat0, 48, 0, A, 0), false, none(), tv(A.d0a, 16, 0, A, 0));
-  conv(9, tv(A.d0a, 16, 0, A, 0), false, none(), tv(A.d0, 16, 0, A, 0));
-  conv(10, tv(A.d0, 16, 0, A, 0), false, tv(A.y, 1, 0, A, 0), none());
+  conv(8, tv(A.cat0, 48, 0, A, 0), none(), tv(A.d0a, 16, 0, A, 0));
+  conv(9, tv(A.d0a, 16, 0, A, 0), none(), tv(A.d0, 16, 0, A, 0));
+  conv(10, tv(A.d0, 16, 0, A, 0), tv(A.y, 1, 0, A, 0), none());
 }
 
 /* Backward of layer l: G (FP32, the gradient of the layer's output after
  * its ReLU mask has been applied), X (its BF16 input); accumulates dW, db
- * and writes the input gradient into GX (FP32) when GX.p != NULL. */
-static void layer_bwd(int l, TV G, TV X, TV GX)
+ * and writes the input gradient into GX (FP32) when GX.p != NULL, zeroed
+ * where M (when given) is not positive. */
+static void layer_bwd(int l, TV G, TV X, TV GX, TV M = none())
 {
   Layer &Y = net->L[l];
   Acts &A = *net->A;
-  long nv = (long) G.nx * G.ny * G.nz;
-  long chunk = chunk_of(nv);
-  long nchunks = (nv + chunk - 1) / chunk;
-  int jobs = Y.taps * (Y.coutp / 16) * (Y.cinp / 16);
-  hipLaunchKernelGGL(conv_wgrad_kernel, dim3((unsigned) nchunks,
-    (unsigned) ((jobs + 3) / 4)), dim3(256), 0, bb_stream, G, Y.cout, X,
-    Y.cin, Y.taps, Y.coutp, Y.cinp, chunk, A.part);
-  ew(sum_chunks_kernel, Y.nw, A.part, Y.nw, (int) nchunks, Y.gw);
-  hipLaunchKernelGGL(bias_grad_kernel, dim3((unsigned) nchunks),
-    dim3(Y.coutp), 0, bb_stream, G, Y.cout, chunk, A.part);
-  ew(sum_chunks_kernel, (long) Y.coutp, A.part, (long) Y.coutp,
-     (int) nchunks, Y.gb);
+  const int nblocks = ((G.nx + CB_X - 1) / CB_X) * ((G.ny + CB_Y - 1) / CB_Y) *
+                      ((G.nz + CB_Z - 1) / CB_Z);
+  const int nci = Y.cinp / 16, nco = Y.coutp / 16;
+  const int nwg = wgrad_chunks(nblocks, nci);
+  const int nchunks = Y.taps == 27 ? nwg : 4 * nwg;
+  float *Pb = A.part + (long) nchunks * Y.nw;
+#define WG(TAPS, NCO) hipLaunchKernelGGL((wgrad_kernel<TAPS, NCO>),           \
+    dim3((unsigned) nwg, (unsigned) nci), dim3(256), 0, bb_stream, G, Y.cout, \
+    X, Y.cinp, nblocks, A.part, Pb)
+  if (Y.taps == 1) WG(1, 1);
+  else if (nco == 4) WG(27, 4);
+  else if (nco == 2) WG(27, 2);
+  else WG(27, 1);
+#undef WG
+  hipLaunchKernelGGL(sum_chunks_kernel,
+    dim3(blocks(Y.nw, 32) + blocks(Y.coutp, 32)), dim3(256), 0, bb_stream,
+    A.part, Y.nw, nchunks, Y.gw, Pb, Y.coutp, nwg, Y.gb);
   if (GX.p) {
     ew(flip_weights_kernel, Y.nw, Y.wb, Y.taps, Y.coutp, Y.cinp, Y.wt);
     conv_launch<float>(G, Y.cout, Y.coutp, Y.wt, Y.taps, (const float *) NULL,
-                       Y.cin, Y.cinp, GX, none(), 0);
+                       Y.cin, Y.cinp, GX, none(), 0, M);
   }
   BB_LAUNCH_CHECK();
-}
-
-static void relu_bwd(TV G, TV Y, int C)
-{
-  ew(relu_bwd_kernel, (long) G.nx * G.ny * G.nz * C, G, Y, C);
 }
 
 /* Backward pass from the output gradient in A.g_y. */
@@ -1034,11 +1220,11 @@ static void backward(void)
   Acts &A = *net->A;
   /* out (1x1, no ReLU): d0 <- */
   layer_bwd(10, tv(A.g_y, 1, 0, A, 0), tv(A.d0, 16, 0, A, 0),
-            tv(A.g_d0, 16, 0, A, 0));
-  relu_bwd(tv(A.g_d0, 16, 0, A, 0), tv(A.d0, 16, 0, A, 0), 16);
+            tv(A.g_d0, 16, 0, A, 0),
+            tv(A.d0, 16, 0, A, 0));
   layer_bwd(9, tv(A.g_d0, 16, 0, A, 0), tv(A.d0a, 16, 0, A, 0),
-            tv(A.g_d0a, 16, 0, A, 0));
-  relu_bwd(tv(A.g_d0a, 16, 0, A, 0), tv(A.d0a, 16, 0, A, 0), 16);
+            tv(A.g_d0a, 16, 0, A, 0),
+            tv(A.d0a, 16, 0, A, 0));
   layer_bwd(8, tv(A.g_d0a, 16, 0, A, 0), tv(A.cat0, 48, 0, A, 0),
             tv(A.g_cat0, 48, 0, A, 0));
   /* cat0 = [up(d1) 0..31 | e0 32..47] */
@@ -1046,8 +1232,8 @@ static void backward(void)
      tv(A.g_d1, 32, 0, A, 1), 32);
   relu_bwd(tv(A.g_d1, 32, 0, A, 1), tv(A.d1, 32, 0, A, 1), 32);
   layer_bwd(7, tv(A.g_d1, 32, 0, A, 1), tv(A.d1a, 32, 0, A, 1),
-            tv(A.g_d1a, 32, 0, A, 1));
-  relu_bwd(tv(A.g_d1a, 32, 0, A, 1), tv(A.d1a, 32, 0, A, 1), 32);
+            tv(A.g_d1a, 32, 0, A, 1),
+            tv(A.d1a, 32, 0, A, 1));
   layer_bwd(6, tv(A.g_d1a, 32, 0, A, 1), tv(A.cat1, 96, 0, A, 1),
             tv(A.g_cat1, 96, 0, A, 1));
   /* cat1 = [up(b1) 0..63 | e1 64..95] */
@@ -1055,8 +1241,8 @@ static void backward(void)
      tv(A.g_b1, 64, 0, A, 2), 64);
   relu_bwd(tv(A.g_b1, 64, 0, A, 2), tv(A.b1, 64, 0, A, 2), 64);
   layer_bwd(5, tv(A.g_b1, 64, 0, A, 2), tv(A.b0, 64, 0, A, 2),
-            tv(A.g_b0, 64, 0, A, 2));
-  relu_bwd(tv(A.g_b0, 64, 0, A, 2), tv(A.b0, 64, 0, A, 2), 64);
+            tv(A.g_b0, 64, 0, A, 2),
+            tv(A.b0, 64, 0, A, 2));
   layer_bwd(4, tv(A.g_b0, 64, 0, A, 2), tv(A.p1, 32, 0, A, 2),
             tv(A.g_p1, 32, 0, A, 2));
   /* e1 gradient: skip path (already in g_cat1[64..95]) + pool path */
@@ -1064,16 +1250,16 @@ static void backward(void)
      tv(A.g_p1, 32, 0, A, 2), 32);
   relu_bwd(tv(A.g_cat1, 96, 64, A, 1), tv(A.cat1, 96, 64, A, 1), 32);
   layer_bwd(3, tv(A.g_cat1, 96, 64, A, 1), tv(A.e1a, 32, 0, A, 1),
-            tv(A.g_e1a, 32, 0, A, 1));
-  relu_bwd(tv(A.g_e1a, 32, 0, A, 1), tv(A.e1a, 32, 0, A, 1), 32);
+            tv(A.g_e1a, 32, 0, A, 1),
+            tv(A.e1a, 32, 0, A, 1));
   layer_bwd(2, tv(A.g_e1a, 32, 0, A, 1), tv(A.p0, 16, 0, A, 1),
             tv(A.g_p0, 16, 0, A, 1));
   ew(pool_bwd_kernel, A.nv[0] * 16, tv(A.g_cat0, 48, 32, A, 0),
      tv(A.g_p0, 16, 0, A, 1), 16);
   relu_bwd(tv(A.g_cat0, 48, 32, A, 0), tv(A.cat0, 48, 32, A, 0), 16);
   layer_bwd(1, tv(A.g_cat0, 48, 32, A, 0), tv(A.e0a, 16, 0, A, 0),
-            tv(A.g_e0a, 16, 0, A, 0));
-  relu_bwd(tv(A.g_e0a, 16, 0, A, 0), tv(A.e0a, 16, 0, A, 0), 16);
+            tv(A.g_e0a, 16, 0, A, 0),
+            tv(A.e0a, 16, 0, A, 0));
   layer_bwd(0, tv(A.g_e0a, 16, 0, A, 0), tv(A.in0, 16, 0, A, 0), none());
 }
 

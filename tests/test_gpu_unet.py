@@ -211,3 +211,37 @@ def test_warm_start_in_solver(case_dir):
     assert eg <= eh * (1 + 1e-6)
     assert lrn < last
     assert pas < hist
+
+
+@pytest.mark.parametrize("dims", [(4, 4, 4), (20, 8, 12), (36, 20, 28),
+                                  (64, 64, 48)])
+def test_gradients_by_volume(net, dims):
+    """Weight and bias gradients where the 16 x 4 x 4 voxel blocks of the
+    gradient kernel do not fill the volume, where one block is all there is
+    at the coarsest level, and where a workgroup takes several blocks (768
+    blocks, more than chunks).  A gradient is a sum of products of an
+    activation and a back-propagated value, each rounded to BF16 (2^-9) once
+    per layer that it passes: 11 layers, 11 * 2^-9 = 2.2e-2."""
+    L, torch = net
+    import unet_ref
+    L.bb_unet_create(1234)          # the solver's teardown destroyed it
+    nv = dims[0] * dims[1] * dims[2]
+    rng = np.random.default_rng(11)
+    x = rng.standard_normal((nv, 2)).astype(np.float32)
+    t = rng.standard_normal(nv).astype(np.float32)
+    assert L.bb_unet_volume(*dims) == 0
+    xd = torch.from_numpy(x).cuda()
+    td = torch.from_numpy(t).cuda()
+    yd = torch.zeros(nv, device="cuda")
+    torch.cuda.synchronize()
+    L.bb_unet_forward(xd.data_ptr(), yd.data_ptr())
+    L.bb_unet_backward(td.data_ptr())
+    L.cuda_block()
+    ws, bs = get_params(L, 0, 1)
+    gws, gbs = get_params(L, 2, 3)
+    _, _, rgw, rgb = unet_ref.grads(ws, bs, x, t, dims)
+    for l in range(11):
+        ew = rel(gws[l], rgw[l])
+        eb = rel(gbs[l][:len(rgb[l])], rgb[l])
+        print(f"{dims} layer {l}: dW rel {ew:.2e}  db rel {eb:.2e}")
+        assert ew <= 2.2e-2 and eb <= 2.2e-2, l
