@@ -36,6 +36,7 @@
 #include <stdint.h>
 
 #include <limits.h>
+#include <string.h>
 #include <type_traits>
 
 #include "bb_common.h"
@@ -145,6 +146,8 @@ struct CGState {
   double relup;       /* mixed form: inner reduction of (r, z) per sweep */
   int q, done, nan_flag, inner_done;
   int lost;           /* a one-launch sweep gave up waiting */
+  int mg;             /* multigrid sweep: rzs holds (r, z) of the V-cycle and
+                         mg_check_kernel alone ends the sweep */
   double alpha;       /* alpha of the last update that left phi alone */
 };
 
@@ -238,6 +241,7 @@ cg_state_init_kernel(const double *__restrict__ bpart,
     st->nan_flag = 0;
     st->inner_done = 0;
     st->lost = 0;
+    st->mg = 0;
     st->alpha = 0.;
   }
 }
@@ -257,6 +261,7 @@ __device__ inline bool cg_continue(CGState *st, const double *__restrict__ rpart
   bool first = blockIdx.x == 0 && threadIdx.x == 0;
   bool stop = s <= st->tol2*st->sp_rhs || isnan(s);
   if (MIXED && !stop) stop = s <= st->relup*st->rz_ref;
+  if (MIXED && st->mg) stop = isnan(s);
   if (stop) {
     if (first) {
       st->rz1 = s;
@@ -2015,6 +2020,8 @@ mx_state_kernel(CGState *st, const double *__restrict__ rpart, long n, int q,
   if (restart) st->rzs[(q + 1) & 1] = s;
 }
 
+#include "bb_mg.h"
+
 /* ------------------------------- driver --------------------------------- */
 static double now_s(void)
 {
@@ -2080,15 +2087,26 @@ static void solve_begin(void)
  * correction 0), from the latest timestep that ran it. */
 #define SWEEP_PASSES 32
 #define SWEEP_OUTER 8
-static int sweep_len[2][SWEEP_PASSES][SWEEP_OUTER];
+enum { SWEEP_PLAIN, SWEEP_MIXED, SWEEP_MG, SWEEP_FORMS };
+static int sweep_len[SWEEP_FORMS][SWEEP_PASSES][SWEEP_OUTER];
+
+/* Iterations to enqueue between the host's checks.  An iteration with a
+ * V-cycle takes some ten times a check's wait, and as many launches that
+ * return at once where it was one too many: two, and the first time as many
+ * as the sweep took a timestep ago. */
+static int batch_of(int form)
+{
+  return form == SWEEP_MG && bb_pcg_batch > 2 ? 2 : bb_pcg_batch;
+}
 
 /* Iterations to enqueue before the first check of a sweep. */
 static int first_batch(int form, int outer)
 {
   const int p = solve_pass;
-  int n = bb_pcg_batch;
+  int n = batch_of(form);
   if (bb_pcg_predict && p >= 0 && p < SWEEP_PASSES && outer < SWEEP_OUTER) {
-    const int m = (int) (0.8 * sweep_len[form][p][outer]);
+    const int m = (int) ((form == SWEEP_MG ? 1. : 0.8) *
+                         sweep_len[form][p][outer]);
     if (m > n) n = m;
   }
   return n;
@@ -2173,6 +2191,11 @@ int bb_resident_spins = 1 << 21;       /* polls (about a microsecond each)
                                           before a wait in it gives up */
 int bb_resident_last = 0;              /* tiles per workgroup of the last
                                           sweep, 0: kernel by kernel */
+int bb_mg = 1;                         /* 1: large grids of the mixed form
+                                          precondition with a V-cycle
+                                          (bb_mg.h); 0: Jacobi always */
+int bb_mg_last = 0;                    /* levels of the last mixed solve, 0:
+                                          Jacobi */
 long bb_pcg_iters_total = 0;           /* PCG iterations over all solves */
 long bb_pcg_solves_total = 0;
 /* Iterations of each solve, in order (entry n % BB_SOLVE_LOG of solve n). */
@@ -2210,6 +2233,35 @@ static void cg_buffers32(void)
   for (int i = 0; i < 5; i++)
     *bufs[i] = (float *) bb_grid_alloc(ddom.cc.n, sizeof(float));
   buf32_n = ddom.cc.n;
+}
+
+/* The multigrid hierarchy of the mixed form: level 0 is the grid itself (its
+ * vectors are _r32 and _mg_z); the others share one allocation. */
+static MGLevel mg_lev[MG_LEVELS];
+static int mg_n = 0;                   /* levels; 0: not for this grid */
+static struct {
+  Grid g;
+  int nx, ny, nz, perx, pery, perz;
+  double hx, hy, hz;
+} mg_key;
+static float *_mg_z = NULL, *_mg_mem = NULL;
+static float *mg_r[MG_LEVELS], *mg_z[MG_LEVELS];
+static uint8_t *mg_m[MG_LEVELS];
+static uint8_t *_mg_mask = NULL;
+static long mg_mask_of = -1;           /* particle mask generation */
+static const uint8_t *mg_fluid = NULL; /* level 0's mask at that time */
+
+static void mg_free(void)
+{
+  bb_grid_free(_mg_z);
+  if (_mg_mem) BB_CHECK(hipFree(_mg_mem));
+  if (_mg_mask) BB_CHECK(hipFree(_mg_mask));
+  _mg_z = _mg_mem = NULL;
+  _mg_mask = NULL;
+  mg_n = 0;
+  mg_mask_of = -1;
+  mg_fluid = NULL;
+  memset(&mg_key, 0, sizeof(mg_key));
 }
 
 /* Set while cuda_PP_cg_noalloc runs: the CG buffers then point into the
@@ -2255,6 +2307,7 @@ void bb_solver_free(void)
   if (_cg_state) BB_CHECK(hipFree(_cg_state));
   if (cg_host) BB_CHECK(hipHostFree(cg_host));
   cg_buffers32_free();
+  mg_free();
   if (_meet) BB_CHECK(hipFree(_meet));
   _meet = NULL;
   resident_cus = 0;
@@ -3006,7 +3059,7 @@ static void pcg_plain(double ts, int warm)
   }
   int q = one_launch ? cg_host->q : 0;
   while (!one_launch && q <= pp_max_iter) {
-    int qend = q + (q == 0 ? first_batch(0, 0) : bb_pcg_batch);
+    int qend = q + (q == 0 ? first_batch(SWEEP_PLAIN, 0) : bb_pcg_batch);
     if (qend > pp_max_iter + 1) qend = pp_max_iter + 1;
     for (int qq = q + 1; qq <= qend; qq++) enqueue_iteration(qq, K, T);
     hipLaunchKernelGGL(cg_check_kernel<false>, dim3(1), dim3(TILE_THREADS),
@@ -3015,7 +3068,7 @@ static void pcg_plain(double ts, int warm)
     fetch_state();
     if (cg_host->done) break;
   }
-  if (cg_host->done) record_sweep(0, 0, cg_host->q);
+  if (cg_host->done) record_sweep(SWEEP_PLAIN, 0, cg_host->q);
   /* a solve that stops right after a PHI_SKIP update: add its term */
   if (!one_launch && cg_host->done && cg_host->q >= 1 &&
       phi_skips(cg_host->q)) {
@@ -3175,17 +3228,190 @@ extern "C" int cuda_PP_cg_noalloc(void)
   return 0;
 }
 
+/* Cells beyond which the mixed form takes the V-cycle.  A solve from phi = 0
+ * to 1e-8 with the Jacobi factor (in one launch where the grid fits) and with
+ * the V-cycle, us: 48^3 with spheres 1779 and 1321, channel 2207 and 1047;
+ * 64^3 2528 and 1361, 3024 and 1219; 96^3 5033 and 1896, 6146 and 1575; 128^3
+ * 7128 and 2186, 10178 and 1682.  It is the faster one below this line too;
+ * there the sweep's iterates are the plain form's. */
+#define MG_MIN_CELLS (1l << 18)
+
+/* The levels of this grid and their vectors; 0: Jacobi.  A direction with an
+ * odd number of cells ends its coarsening, so a grid whose sizes hold few
+ * factors of two may not reach MG_LAST_MAX cells and keeps Jacobi. */
+static int mg_setup(const Coef &K)
+{
+  const long cells = (long) ddom.nx * ddom.ny * ddom.nz;
+  if (!bb_mg || bb_mixed_restart || cells <= MG_MIN_CELLS ||
+      ddom.cc.n > INT_MAX)
+    return 0;
+  auto key = mg_key;
+  memset(&key, 0, sizeof(key));
+  key.g = ddom.cc;
+  key.nx = ddom.nx; key.ny = ddom.ny; key.nz = ddom.nz;
+  key.perx = ddom.perx; key.pery = ddom.pery; key.perz = ddom.perz;
+  key.hx = K.idx2; key.hy = K.idy2; key.hz = K.idz2;
+  if (memcmp(&key, &mg_key, sizeof(key)) != 0) {
+    mg_free();
+    mg_key = key;
+    MGLevel L = {};
+    L.nx = ddom.nx; L.ny = ddom.ny; L.nz = ddom.nz;
+    L.sy = (int) ddom.cc.sy; L.sz = (int) ddom.cc.sz;
+    L.perx = ddom.perx; L.pery = ddom.pery; L.perz = ddom.perz;
+    L.hx = (float) K.idx2; L.hy = (float) K.idy2; L.hz = (float) K.idz2;
+    int n = 1;
+    mg_lev[0] = L;
+    while (n < MG_LEVELS && (long) L.nx * L.ny * L.nz > MG_LAST) {
+      /* 1/h^2 at least that of 1.5 times the smallest spacing */
+      const float cut = fmaxf(L.hx, fmaxf(L.hy, L.hz)) / 2.25f;
+      const int cx = L.hx >= cut && L.nx % 2 == 0 && L.nx >= 8;
+      const int cy = L.hy >= cut && L.ny % 2 == 0 && L.ny >= 8;
+      const int cz = L.hz >= cut && L.nz % 2 == 0 && L.nz >= 8;
+      if (!(cx | cy | cz)) break;
+      if (cx) { L.nx /= 2; L.hx /= 4; }
+      if (cy) { L.ny /= 2; L.hy /= 4; }
+      if (cz) { L.nz /= 2; L.hz /= 4; }
+      L.sy = (L.nx + 31) / 32 * 32;
+      L.sz = L.sy * L.ny;
+      mg_lev[n++] = L;
+    }
+    if ((long) L.nx * L.ny * L.nz > MG_LAST_MAX) return 0;
+    mg_lev[n - 1].sy = L.nx;
+    mg_lev[n - 1].sz = L.nx * L.ny;
+    /* the grid's own rows start on 128 bytes (bb_grid_alloc), the others'
+     * strides are multiples of 32 but for the last level's */
+    for (int l = 0; l < n; l++)
+      mg_lev[l].vec = mg_lev[l].nx % 4 == 0 && mg_lev[l].sy % 4 == 0 &&
+                      mg_lev[l].sz % 4 == 0;
+    /* runs of four also in a last level that keeps the row */
+    for (int l = 0; l + 1 < n; l++)
+      if (mg_lev[l + 1].nx == mg_lev[l].nx) mg_lev[l].vec &= mg_lev[l + 1].vec;
+    long tot = 0, off[MG_LEVELS];
+    for (int l = 1; l < n; l++) {
+      off[l] = tot;
+      tot += ((long) mg_lev[l].sz * mg_lev[l].nz + 31) / 32 * 32;
+    }
+    BB_CHECK(hipMalloc((void **) &_mg_mem, 2 * tot * sizeof(float)));
+    BB_CHECK(hipMalloc((void **) &_mg_mask, tot));
+    _mg_z = (float *) bb_grid_alloc(ddom.cc.n, sizeof(float));
+    for (int l = 1; l < n; l++) {
+      mg_r[l] = _mg_mem + off[l];
+      mg_z[l] = _mg_mem + tot + off[l];
+      mg_m[l] = _mg_mask + off[l];
+    }
+    mg_n = n;
+  }
+  if (!mg_n) return 0;
+  const uint8_t *fm = fluid_mask();
+  if (mg_mask_of != bb_mask_gen || mg_fluid != fm) {
+    if (!rows_aligned(_r32, 4, 16) || !rows_aligned(_mg_z, 4, 16) ||
+        (fm && !rows_aligned(fm, 1, 4)))
+      mg_lev[0].vec = 0;
+    mg_lev[0].m = fm ? fm + gidx(ddom.cc, 1, 1, 1) : NULL;
+    for (int l = 1; l < mg_n; l++) {
+      const MGLevel &F = mg_lev[l - 1];
+      MGLevel &C = mg_lev[l];
+      C.m = fm ? mg_m[l] : NULL;
+      if (fm)
+        hipLaunchKernelGGL(mg_mask_kernel, dim3((unsigned) ((C.nx + 63) / 64),
+          (unsigned) ((C.ny + 3) / 4), (unsigned) C.nz), dim3(256), 0,
+          bb_stream, F, C, F.nx != C.nx, F.ny != C.ny, F.nz != C.nz, mg_m[l]);
+    }
+    BB_LAUNCH_CHECK();
+    mg_mask_of = bb_mask_gen;
+    mg_fluid = fm;
+  }
+  return mg_n;
+}
+
+/* z = M^-1 r: one V-cycle on _r32 into _mg_z, with the workgroups' partials
+ * of (r, z) in `part`.  The singular system's last level takes the mean out. */
+static void mg_cycle(double *part)
+{
+  const long o0 = gidx(ddom.cc, 1, 1, 1);
+  const int last = mg_n - 1;
+  auto R = [&](int l) { return l ? mg_r[l] : _r32 + o0; };
+  auto Z = [&](int l) { return l ? mg_z[l] : _mg_z + o0; };
+  auto dirs = [&](int l) {
+    return (mg_lev[l].nx != mg_lev[l + 1].nx) +
+           2 * (mg_lev[l].ny != mg_lev[l + 1].ny) +
+           4 * (mg_lev[l].nz != mg_lev[l + 1].nz);
+  };
+#define MG_VEC(KERNEL, l, X, Y, Z, ...)                                      \
+  if (mg_lev[l].vec)                                                          \
+    hipLaunchKernelGGL((KERNEL<X, Y, Z, true>), __VA_ARGS__);                 \
+  else hipLaunchKernelGGL((KERNEL<X, Y, Z, false>), __VA_ARGS__)
+#define MG_DIRS(KERNEL, l, ...)                                               \
+  switch (dirs(l)) {                                                          \
+    case 1: MG_VEC(KERNEL, l, true, false, false, __VA_ARGS__); break;        \
+    case 2: MG_VEC(KERNEL, l, false, true, false, __VA_ARGS__); break;        \
+    case 3: MG_VEC(KERNEL, l, true, true, false, __VA_ARGS__); break;         \
+    case 4: MG_VEC(KERNEL, l, false, false, true, __VA_ARGS__); break;        \
+    case 5: MG_VEC(KERNEL, l, true, false, true, __VA_ARGS__); break;         \
+    case 6: MG_VEC(KERNEL, l, false, true, true, __VA_ARGS__); break;         \
+    default: MG_VEC(KERNEL, l, true, true, true, __VA_ARGS__); break;         \
+  }
+  for (int l = 0; l < last; l++) {
+    const MGLevel &F = mg_lev[l], &C = mg_lev[l + 1];
+    const int zc = mg_planes(F);
+    MG_DIRS(mg_down_kernel, l, dim3(mg_groups(F, zc)), dim3(TILE_THREADS), 0,
+      bb_stream, _cg_state, F, C, zc, R(l), R(l + 1))
+  }
+  {
+    const MGLevel &L = mg_lev[last];
+    const float lmax = 4.f * (L.hx + L.hy + L.hz);
+    auto mode = [](float h, int n, int per) {
+      return n > 1 ? h * (2. - 2. * cos((per ? 2. : 1.) * M_PI / n)) : HUGE_VAL;
+    };
+    const float lmin = (float) fmin(mode(L.hx, L.nx, L.perx),
+      fmin(mode(L.hy, L.ny, L.pery), mode(L.hz, L.nz, L.perz)));
+    int degree = (int) ceilf(0.9f * sqrtf(lmax / lmin));
+    degree = degree < 8 ? 8 : (degree > 32 ? 32 : degree);
+    const int singular = mg_lev[0].m == NULL;
+    if (L.nx * L.ny * L.nz <= 4096)
+      hipLaunchKernelGGL(mg_last_kernel<4>, dim3(1), dim3(1024), 0, bb_stream,
+        _cg_state, L, lmin, lmax, degree, singular, R(last), Z(last));
+    else
+      hipLaunchKernelGGL(mg_last_kernel<16>, dim3(1), dim3(1024), 0, bb_stream,
+        _cg_state, L, lmin, lmax, degree, singular, R(last), Z(last));
+  }
+  for (int l = last - 1; l >= 0; l--) {
+    const MGLevel &F = mg_lev[l], &C = mg_lev[l + 1];
+    const int zc = mg_planes(F);
+    MG_DIRS(mg_up_kernel, l, dim3(mg_groups(F, zc)), dim3(TILE_THREADS), 0,
+      bb_stream, _cg_state, F, C, zc, R(l), Z(l + 1), Z(l), l ? NULL : part)
+  }
+#undef MG_DIRS
+#undef MG_VEC
+  BB_LAUNCH_CHECK();
+}
+
 /* Enqueue inner iteration q of the mixed form (FP32 vectors); `first`
- * starts a new Krylov space (p = z). */
+ * starts a new Krylov space (p = z).  With `mg` z comes from a V-cycle: the
+ * search then takes it for r under a Jacobi factor of one, and goes by its
+ * (r, z); the update's partials of (r, D^-1 r) end the sweep. */
 static void enqueue_iteration32(int q, bool first, const CoefT<float> &K,
-  const InvMT<float> &T)
+  const InvMT<float> &T, bool mg)
 {
   const long nt = n_tiles(ddom);
   float *pnew = (q & 1) ? _p32a : _p32b;
   float *pold = (q & 1) ? _p32b : _p32a;
+  if (mg) {
+    hipLaunchKernelGGL(mg_check_kernel, dim3(1), dim3(TILE_THREADS), 0,
+      bb_stream, _cg_state, q - 1, _part_r, nt);
+    mg_cycle(_part_w1);
+  }
   bb_kt_q = q;
   bb_kt_begin(KT_SPMV32);
-  if (first)
+  if (mg) {
+    InvMT<float> one;
+    for (int i = 0; i < 27; i++) one.v[i] = 1.f;
+    double *const part_r = _part_r;
+    _part_r = _part_w1;
+    launch_group<false, float, true>(K, one, q, mg_groups(mg_lev[0],
+      mg_planes(mg_lev[0])), _mg_z, pold, pnew, _Ap32);
+    _part_r = part_r;
+  } else if (first)
     launch_group<true, float, true>(K, T, q, nt, _r32, pold, pnew, _Ap32);
   else
     launch_group<false, float, true>(K, T, q, nt, _r32, pold, pnew, _Ap32);
@@ -3244,6 +3470,8 @@ static void pcg_mixed(double ts, int warm)
   }
   cg_buffers();
   cg_buffers32();
+  const int mg = bb_mg_last = mg_setup(K);
+  const int form = mg ? SWEEP_MG : SWEEP_MIXED;
 
   auto start = [&](int from_phi) {
     if (from_phi) {
@@ -3257,6 +3485,11 @@ static void pcg_mixed(double ts, int warm)
     hipLaunchKernelGGL(cg_state_init_kernel, dim3(1), dim3(TILE_THREADS), 0,
       bb_stream, _part_p, _part_r, nt, _cg_state, pp_residual*pp_residual,
       pp_inner_tol*pp_inner_tol);
+    if (mg) {
+      hipLaunchKernelGGL(mg_start_kernel, dim3(1), dim3(1), 0, bb_stream,
+        _cg_state);
+      hipLaunchKernelGGL(mx_zero_kernel, TILES_LAUNCH, ddom, _p32b);
+    }
     BB_LAUNCH_CHECK();
   };
   start(warm);
@@ -3283,7 +3516,17 @@ static void pcg_mixed(double ts, int warm)
   /* the FP64 correction after the sweep that ended with iteration `at`, and
    * the state it leaves */
   auto correct = [&](int at) {
-    hipLaunchKernelGGL(mx_fold_kernel, TILES_LAUNCH, ddom, _phi, _e32);
+    if (mg && !fluid_mask()) {
+      const double sd =
+        K.idx2*(2.*ddom.nx - (ddom.perx ? 0 : 2))*ddom.ny*ddom.nz +
+        K.idy2*(2.*ddom.ny - (ddom.pery ? 0 : 2))*ddom.nx*ddom.nz +
+        K.idz2*(2.*ddom.nz - (ddom.perz ? 0 : 2))*ddom.nx*ddom.ny;
+      hipLaunchKernelGGL(mg_mean_kernel, TILES_LAUNCH, ddom, T, _e32,
+        _part_w1);
+      hipLaunchKernelGGL(mg_fold_kernel, TILES_LAUNCH, ddom, _part_w1, nt, sd,
+        _phi, _e32);
+    } else
+      hipLaunchKernelGGL(mx_fold_kernel, TILES_LAUNCH, ddom, _phi, _e32);
     hipLaunchKernelGGL(mx_residual_kernel, TILES_LAUNCH, ddom, K, T, _phi,
       _rhs_p, fluid_mask(), _r32, _part_r);
     hipLaunchKernelGGL(mx_state_kernel, dim3(1), dim3(TILE_THREADS), 0,
@@ -3291,7 +3534,7 @@ static void pcg_mixed(double ts, int warm)
     BB_LAUNCH_CHECK();
     fetch_state();
   };
-  int ntw = resident_tiles(sizeof(float));
+  int ntw = mg ? 0 : resident_tiles(sizeof(float));
   while (!done && q <= pp_max_iter && nouter <= pp_max_iter) {
     if (ntw) {
       /* a sweep, its correction and the stopping test; one host read */
@@ -3319,7 +3562,7 @@ static void pcg_mixed(double ts, int warm)
         first_q = pair_base32 = 1;
         continue;
       }
-      record_sweep(1, nouter - 1, cg_host->q - q);
+      record_sweep(SWEEP_MIXED, nouter - 1, cg_host->q - q);
       q = sweep0 = cg_host->q;
       pair_base32 = q + 1;
       nouter++;
@@ -3327,19 +3570,24 @@ static void pcg_mixed(double ts, int warm)
       if (bb_mixed_restart) first_q = q + 1;
       continue;
     }
-    int qend = q + (q == sweep0 ? first_batch(1, nouter - 1) : bb_pcg_batch);
+    int qend = q + (q == sweep0 ? first_batch(form, nouter - 1)
+                                : batch_of(form));
     if (qend > pp_max_iter + 1) qend = pp_max_iter + 1;
     for (int qq = q + 1; qq <= qend; qq++)
-      enqueue_iteration32(qq, qq == first_q, K32, T32);
-    hipLaunchKernelGGL(cg_check_kernel<true>, dim3(1), dim3(TILE_THREADS),
-      0, bb_stream, _cg_state, qend, _part_r, nt);
+      enqueue_iteration32(qq, qq == first_q, K32, T32, mg != 0);
+    if (mg)
+      hipLaunchKernelGGL(mg_check_kernel, dim3(1), dim3(TILE_THREADS), 0,
+        bb_stream, _cg_state, qend, _part_r, nt);
+    else
+      hipLaunchKernelGGL(cg_check_kernel<true>, dim3(1), dim3(TILE_THREADS),
+        0, bb_stream, _cg_state, qend, _part_r, nt);
     fetch_state();
     if (!cg_host->inner_done) {
       q = qend;
       continue;
     }
     q = cg_host->q;
-    record_sweep(1, nouter - 1, q - sweep0);
+    record_sweep(form, nouter - 1, q - sweep0);
     sweep0 = q;
     /* e must be whole before the fold: add a skipped update's term */
     if (q >= pair_base32 && phi_skips32(q))

@@ -1,0 +1,131 @@
+"""The V-cycle that preconditions the mixed form's sweeps on large grids
+(bb_mg.h) against the Jacobi factor: the same timestep with both.  Grids whose
+levels take every path of the level kernels: runs of four cells and single
+ones, tiles that end inside a run, each combination of coarsened directions
+that a spacing can ask for, walls and periodic faces, a last level of more than
+4096 cells, particles."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import bbconfig
+import bbhip
+
+pytestmark = pytest.mark.gpu
+
+
+def box(n, per, h):
+    """Walls, one of them moving, where a direction is not periodic."""
+    P = ("PERIODIC",)
+    face = {f: P if per["WESNBT".index(f) // 2] else None for f in "WESNBT"}
+    wall = ("DIRICHLET", 0.0, 0.0)
+    vel = {c: {f: face[f] or wall for f in "WESNBT"} for c in "uvw"}
+    for c, f in (("v", "T"), ("w", "E"), ("u", "N")):
+        if not face[f]:
+            vel[c][f] = ("DIRICHLET", 0.4, 0.0)
+    return dict(n=n, lo=(0.0, 0.0, 0.0),
+                hi=tuple(a * m for a, m in zip(h, n)), rho_f=1.0, nu=0.01,
+                duration=1.0, pp_max_iter=100000, pp_residual=1e-8,
+                p_bc={f: face[f] or ("NEUMANN", 0.0) for f in "WESNBT"},
+                vel_bc=vel, init_cond="QUIESCENT",
+                extensions={"fixed_dt": 1e-3, "perturb": (7, 0.2),
+                            "pp_precision": "MIXED"})
+
+
+def run(case_dir, kw, parts, mg):
+    lib = bbhip.load()
+    on = ctypes.c_int.in_dll(lib, "bb_mg")
+    saved = on.value
+    on.value = mg
+    try:
+        bbconfig.write_case(case_dir, **kw)
+        if parts:
+            bbconfig.write_parts(case_dir, parts)
+        with bbhip.Simulation(case_dir, kw["n"]) as s:
+            s.step()
+            s.pull()
+            return dict(
+                s.pp_stats(), dt=s.scalar("dt"),
+                levels=ctypes.c_int.in_dll(lib, "bb_mg_last").value,
+                **{f: np.array(s.field(f)) for f in ("u", "v", "w", "phi")})
+    finally:
+        on.value = saved
+
+
+def inner(a, n):
+    """The cells (faces) of the domain, without the ghosts."""
+    lo = [(s - m) // 2 for s, m in zip(a.shape, n)]
+    return a[tuple(slice(l, l + m) for l, m in zip(lo, n))]
+
+
+def difference_bound(out, h, low):
+    """Both solves leave residuals with (r, D^-1 r) <= 1e-16 (b, b), so their
+    difference e has A e = r1 - r2 and (A e, e) <= (2e-8)^2 (b, b) / low, low
+    the smallest eigenvalue of D^-1 A (without the constant).  The velocities
+    differ by dt / rho times the differences of e, whose squares sum to
+    (A e, e)."""
+    return out["dt"] * 2e-8 * np.sqrt(out["sp_rhs"] / low)
+
+
+def velocity_difference(a, b, n):
+    return np.sqrt(sum(np.sum((inner(a[f], n) - inner(b[f], n)) ** 2)
+                       for f in "uvw"))
+
+
+@pytest.mark.parametrize("n,per,h,levels", [
+    ((128, 96, 96), (1, 1, 1), (1.0, 1.0, 1.0), 4),
+    ((216, 72, 72), (0, 1, 0), (1.0, 0.8, 1.2), 4),
+    ((200, 200, 28), (0, 0, 1), (1.0, 1.0, 1.0), 4),
+    ((129, 96, 96), (1, 0, 0), (20.0, 1.0, 1.0), 5),
+    ((64, 256, 72), (1, 0, 1), (1.0, 0.2, 1.0), 6),
+    ((512, 48, 48), (1, 1, 0), (0.2, 1.0, 1.0), 6),
+    ((48, 48, 512), (0, 0, 0), (1.0, 0.45, 0.2), 5),
+    ((130, 96, 96), (1, 1, 1), (1.0, 1.0, 1.0), 0),
+    ((100, 96, 96), (1, 0, 1), (1.0, 1.0, 1.0), 4),
+    ((64, 64, 64), (1, 1, 1), (1.0, 1.0, 1.0), 0)])
+def test_same_step(case_dir, n, per, h, levels):
+    """levels: 0 where Jacobi stays (sizes with too few factors of two, no more
+    than 2^18 cells)."""
+    kw = box(n, per, h)
+    ref, out = run(case_dir, kw, None, 0), run(case_dir, kw, None, 1)
+    print("levels", out["levels"], "iterations", ref["niter"], out["niter"])
+    assert ref["levels"] == 0 and bool(out["levels"]) == bool(levels)
+    if not levels:
+        assert ref["niter"] == out["niter"]
+        return
+    assert out["levels"] == levels
+    assert out["resid"] <= 1e-8 and out["niter"] <= 30 < ref["niter"]
+    c = [1.0 / a ** 2 for a in h]
+    low = min((2 - 2 * np.cos((2 if p else 1) * np.pi / m)) * a
+              for a, m, p in zip(c, n, per)) / (2 * sum(c))
+    assert velocity_difference(ref, out, n) <= difference_bound(out, h, low)
+    # the constant that the singular system leaves open: the mean of D phi is
+    # 0 in both, to the FP32 rounding of the sweeps' phi (8 units)
+    D = sum(a * np.where(
+        (np.arange(m) % (m - 1) == 0) & (not p), 1.0, 2.0).reshape(
+            [-1 if d == i else 1 for d in range(3)])
+        for i, (a, m, p) in enumerate(zip(c, n, per)))
+    for s in (ref, out):
+        phi = inner(s["phi"], n)
+        assert abs(np.sum(D * phi)) <= 8 * 2.0 ** -24 * np.sum(D * np.abs(phi))
+
+
+@pytest.mark.parametrize("n,walls", [((128, 96, 96), ""), ((144, 96, 80), "z")])
+def test_same_step_particles(case_dir, n, walls):
+    """Particle cells masked on every level.  The smallest eigenvalue is that
+    of absorbing spheres in a box, at least the one of a single sphere: 4 pi a
+    / V (its capacity), over 6 for D^-1.  Twice the bound for the particles'
+    answer to the difference."""
+    a = 8.0
+    kw, parts = bbconfig.sediment(n=n, nparts=3, a=a, seed=13, walls=walls)
+    for P, c in zip(parts, ((20., 20., 20.), (64., 50., 53.), (94., 70., 45.))):
+        P.update(x=c[0], y=c[1], z=c[2])
+    kw["extensions"] = {"pp_precision": "MIXED"}
+    ref, out = run(case_dir, kw, parts, 0), run(case_dir, kw, parts, 1)
+    print("levels", out["levels"], "iterations", ref["niter"], out["niter"])
+    assert ref["levels"] == 0 and out["levels"] > 1
+    assert out["resid"] <= 1e-8 and out["niter"] <= 30 < ref["niter"]
+    low = 4 * np.pi * a / np.prod(n) / 6
+    assert velocity_difference(ref, out, n) <= \
+        2 * difference_bound(out, (1., 1., 1.), low)
