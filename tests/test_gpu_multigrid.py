@@ -122,7 +122,8 @@ def test_same_step_particles(case_dir, n, walls):
     for P, c in zip(parts, ((20., 20., 20.), (64., 50., 53.), (94., 70., 45.))):
         P.update(x=c[0], y=c[1], z=c[2])
     kw["extensions"] = {"pp_precision": "MIXED"}
-    ref, out = run(case_dir, kw, parts, 0), run(case_dir, kw, parts, 1)
+    assert run(case_dir, kw, parts, 1)["levels"] == 0       # on request only
+    ref, out = run(case_dir, kw, parts, 0), run(case_dir, kw, parts, 2)
     print("levels", out["levels"], "iterations", ref["niter"], out["niter"])
     assert ref["levels"] == 0 and out["levels"] > 1
     assert out["resid"] <= 1e-8 and out["niter"] <= 30 < ref["niter"]
