@@ -484,7 +484,7 @@ conv_lds_kernel(TV X, int cin_pad, const uint16_t *__restrict__ W,
  * The kernel that this replaces gathered every operand element by itself from
  * memory, 16 voxels per product, once per tap, and summed the bias in a pass
  * of one thread per channel: 219 and 51 us per layer (mean over the eleven
- * layers of a 64^3 crop) where this one takes 13 to 21.  What bounds it now is
+ * layers of a 64^3 crop) where this one takes 11 to 35.  What bounds it now is
  * the 18 x 6 x 6 staging (2.5 times the voxels of a block) behind one barrier
  * per block; four training steps of that crop went from 20.6 to 4.2 ms. */
 __device__ inline u16x4 lds_read_tr(const uint16_t *p)
@@ -657,7 +657,7 @@ wgrad_kernel(TV G, int cout, TV X, int cin_pad, int nblocks,
 /* gw and gb: the sums of the partials over their chunks, 32 elements and
  * eight runs of chunks per workgroup (each run in chunk order, then the
  * runs).  One thread per element, all chunks in turn, took 55 us per layer;
- * this takes 8 where the partials take 1 to 5 to read. */
+ * this takes 8 to 27 where the partials take 1 to 5 to read. */
 __global__ void __launch_bounds__(256)
 sum_chunks_kernel(const float *__restrict__ P, long n, int nchunks,
   float *__restrict__ gw, const float *__restrict__ Pb, int nb, int nchunksb,
