@@ -608,7 +608,10 @@ mg_last_kernel(const CGState *st, MGLevel L, float lmin, float lmax,
   if (st->done | st->inner_done) return;
   const int n = L.nx * L.ny * L.nz, t = threadIdx.x, s2 = L.nx * L.ny;
   float res[Q], x[Q], d[Q];
-  int at[Q];                          /* cx, cy, cz in 10 bits each, fluid */
+  /* which of a cell's six neighbours lie in the box (bits 0 to 5: west, east,
+   * south, north, below, above), and bit 6 in a fluid cell; a level of MG_LAST_MAX
+   * cells may be that long in one direction */
+  int at[Q];
   float sum = 0.f;
 #pragma unroll
   for (int q = 0; q < Q; q++) {
@@ -616,8 +619,10 @@ mg_last_kernel(const CGState *st, MGLevel L, float lmin, float lmax,
     const bool on = c < n && (L.m == NULL || L.m[c]);
     res[q] = on ? r[c] : 0.f;
     sum += res[q];
-    at[q] = c % L.nx | ((c / L.nx) % L.ny) << 10 | (c / s2) << 20 |
-            (on ? 1 << 30 : 0);
+    const int cx = c % L.nx, cy = (c / L.nx) % L.ny, cz = c / s2;
+    at[q] = (cx > 0) | (cx < L.nx - 1) << 1 | (cy > 0) << 2 |
+            (cy < L.ny - 1) << 3 | (cz > 0) << 4 | (cz < L.nz - 1) << 5 |
+            on << 6;
   }
   if (singular) {
     for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, WAVE);
@@ -627,7 +632,7 @@ mg_last_kernel(const CGState *st, MGLevel L, float lmin, float lmax,
     for (int i = 0; i < 16; i++) tot += s_sum[i];
 #pragma unroll
     for (int q = 0; q < Q; q++)
-      if (at[q] >> 30) res[q] -= tot / (float) n;
+      if (at[q] >> 6) res[q] -= tot / (float) n;
   }
   const float th = 0.5f * (lmax + lmin), de = 0.5f * (lmax - lmin);
   const float sg = th / de;
@@ -646,18 +651,17 @@ mg_last_kernel(const CGState *st, MGLevel L, float lmin, float lmax,
 #pragma unroll
     for (int q = 0; q < Q; q++) {
       const int i = t + 1024 * q;
-      const int cx = at[q] & 1023, cy = (at[q] >> 10) & 1023,
-                cz = (at[q] >> 20) & 1023;
+      const int f = at[q];
       const float c = d[q];
       float a = 0.f;
-      if (at[q] >> 30) {
+      if (f >> 6) {
         /* beyond a wall: the cell itself, no difference */
-        const int w = cx > 0 ? i - 1 : (L.perx ? i + L.nx - 1 : i);
-        const int e = cx < L.nx - 1 ? i + 1 : (L.perx ? i - L.nx + 1 : i);
-        const int s = cy > 0 ? i - L.nx : (L.pery ? i + s2 - L.nx : i);
-        const int o = cy < L.ny - 1 ? i + L.nx : (L.pery ? i - s2 + L.nx : i);
-        const int b = cz > 0 ? i - s2 : (L.perz ? i + n - s2 : i);
-        const int u = cz < L.nz - 1 ? i + s2 : (L.perz ? i - n + s2 : i);
+        const int w = f & 1 ? i - 1 : (L.perx ? i + L.nx - 1 : i);
+        const int e = f & 2 ? i + 1 : (L.perx ? i - L.nx + 1 : i);
+        const int s = f & 4 ? i - L.nx : (L.pery ? i + s2 - L.nx : i);
+        const int o = f & 8 ? i + L.nx : (L.pery ? i - s2 + L.nx : i);
+        const int b = f & 16 ? i - s2 : (L.perz ? i + n - s2 : i);
+        const int u = f & 32 ? i + s2 : (L.perz ? i - n + s2 : i);
         a = L.hx * ((c - s_d[w]) + (c - s_d[e]))
           + L.hy * ((c - s_d[s]) + (c - s_d[o]))
           + L.hz * ((c - s_d[b]) + (c - s_d[u]));

@@ -111,6 +111,31 @@ def test_same_step(case_dir, n, per, h, levels):
         assert abs(np.sum(D * phi)) <= 8 * 2.0 ** -24 * np.sum(D * np.abs(phi))
 
 
+@pytest.mark.parametrize("n,per,h", [
+    ((1153, 2, 128), (1, 1, 1), (16.0, 16.0, 1.0)),
+    ((1153, 2, 128), (0, 0, 0), (16.0, 16.0, 1.0)),
+    ((2, 1153, 128), (1, 0, 1), (16.0, 16.0, 1.0)),
+    ((2, 128, 1153), (0, 1, 1), (16.0, 1.0, 16.0)),
+    ((128, 2, 1027), (1, 1, 0), (1.0, 16.0, 16.0))])
+def test_long_last_level(case_dir, n, per, h):
+    """A last level of more than 1024 cells in one direction (1153 x 2 x 4 and
+    its like), against the plain form: FP32 sweeps with the Jacobi factor
+    stall on such boxes.  Their condition number is up to 1.6e6 on the last
+    level; its polynomial of degree 32 leaves 1 / (4 32^2) of it, 400, which
+    is some 190 iterations (sqrt(400) / 2 times ln(2e8))."""
+    kw = box(n, per, h)
+    out = run(case_dir, kw, None, 1)
+    kw["extensions"]["pp_precision"] = "PLAIN"
+    ref = run(case_dir, kw, None, 1)
+    print("levels", out["levels"], "iterations", ref["niter"], out["niter"])
+    assert out["levels"] > 1
+    assert out["resid"] <= 1e-8 and out["niter"] <= 200
+    c = [1.0 / a ** 2 for a in h]
+    low = min((2 - 2 * np.cos((2 if p else 1) * np.pi / m)) * a
+              for a, m, p in zip(c, n, per)) / (2 * sum(c))
+    assert velocity_difference(ref, out, n) <= difference_bound(out, h, low)
+
+
 @pytest.mark.parametrize("n,walls", [((128, 96, 96), ""), ((144, 96, 80), "z")])
 def test_same_step_particles(case_dir, n, walls):
     """Particle cells masked on every level.  The smallest eigenvalue is that
