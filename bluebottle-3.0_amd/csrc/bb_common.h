@@ -77,6 +77,8 @@ struct Grid {
 #define GRID_ROW_ALIGN 32             /* row stride multiple (elements) */
 #define GRID_ORIGIN 31                /* leading elements of an array */
 void *bb_grid_alloc(long n, size_t esize);
+void *bb_grid_try_alloc(long n, size_t esize);
+void *bb_try_alloc(size_t bytes);
 void bb_grid_free(void *p);
 
 __host__ __device__ inline long gidx(const Grid &G, int i, int j, int k)

@@ -82,14 +82,40 @@ static Grid make_grid(const grid_info &G)
 #define GRID_ALLOCS 512
 static struct { void *user, *raw; } grid_tab[GRID_ALLOCS];
 
-void *bb_grid_alloc(long n, size_t esize)
+/* Buffers that only make a solve faster, and that it does without where they
+ * do not fit: NULL instead of an exit.  They come in the first solve, before
+ * the arrays of the learned guess (nine of the grid in FP64 and the network's),
+ * and one may take 1/32 of the free memory, so that a run that fits without
+ * them still does. */
+long bb_optional_max = -1;             /* bytes of one at most; -1: only the
+                                          bound above */
+
+void *bb_try_alloc(size_t bytes)
 {
-  size_t bytes = (size_t) (n + GRID_ORIGIN + 1) * esize;
-  char *raw = NULL;
-  BB_CHECK(hipMalloc((void **) &raw, bytes));
+  void *p = NULL;
+  size_t left = 0, all = 0;
+  if (bb_optional_max >= 0 && bytes > (size_t) bb_optional_max) return NULL;
+  BB_CHECK(hipMemGetInfo(&left, &all));
+  if (bytes > left / 32) return NULL;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e == hipSuccess) return p;
+  (void) hipGetLastError();
+  if (e != hipErrorOutOfMemory) BB_CHECK(e);
+  return NULL;
+}
+
+static size_t grid_bytes(long n, size_t esize)
+{
+  return (size_t) (n + GRID_ORIGIN + 1) * esize;
+}
+
+/* The cleared grid array in `raw`. */
+static void *grid_array(void *raw, long n, size_t esize)
+{
+  const size_t bytes = grid_bytes(n, esize);
   BB_CHECK(hipMemset(raw, 0, bytes));
   gpumem += bytes;
-  void *user = raw + (size_t) GRID_ORIGIN * esize;
+  void *user = (char *) raw + (size_t) GRID_ORIGIN * esize;
   for (int i = 0; i < GRID_ALLOCS; i++)
     if (grid_tab[i].user == NULL) {
       grid_tab[i].user = user;
@@ -98,6 +124,19 @@ void *bb_grid_alloc(long n, size_t esize)
     }
   fprintf(stderr, "bb_grid_alloc: more than %d grid arrays\n", GRID_ALLOCS);
   exit(EXIT_FAILURE);
+}
+
+void *bb_grid_alloc(long n, size_t esize)
+{
+  void *raw = NULL;
+  BB_CHECK(hipMalloc(&raw, grid_bytes(n, esize)));
+  return grid_array(raw, n, esize);
+}
+
+void *bb_grid_try_alloc(long n, size_t esize)
+{
+  void *raw = bb_try_alloc(grid_bytes(n, esize));
+  return raw ? grid_array(raw, n, esize) : NULL;
 }
 
 void bb_grid_free(void *p)

@@ -2969,14 +2969,18 @@ static hipError_t resident_launch(const CoefT<V> &K, const InvMT<V> &T,
 }
 
 /* One sweep in one launch, `nt` tiles per workgroup; false: it could not be
- * launched, and this simulation does not try again. */
+ * launched (or its slots not allocated), and this simulation does not try
+ * again. */
 template <typename V, bool MIXED>
 static bool resident_sweep(int nt, const CoefT<V> &K, const InvMT<V> &T,
   Sweep<V> S)
 {
   if (!_meet)
-    BB_CHECK(hipMalloc((void **) &_meet,
-      MEET_SETS * MEET_SLOTS * sizeof(u64)));
+    _meet = (u64 *) bb_try_alloc(MEET_SETS * MEET_SLOTS * sizeof(u64));
+  if (!_meet) {
+    resident_cus = -1;
+    return false;
+  }
   S.slots = _meet;
   S.fluid = fluid_mask();
   S.rpart = _part_r;
@@ -3237,9 +3241,10 @@ extern "C" int cuda_PP_cg_noalloc(void)
  * there the sweep's iterates are the plain form's. */
 #define MG_MIN_CELLS (1l << 18)
 
-/* The levels of this grid and their vectors; 0: Jacobi.  A direction with an
- * odd number of cells ends its coarsening, so a grid whose sizes hold few
- * factors of two may not reach MG_LAST_MAX cells and keeps Jacobi. */
+/* The levels of this grid and their vectors; 0: Jacobi, also where the vectors
+ * do not fit in memory.  A direction with an odd number of cells ends its
+ * coarsening, so a grid whose sizes hold few factors of two may not reach
+ * MG_LAST_MAX cells and keeps Jacobi. */
 static int mg_setup(const Coef &K)
 {
   const long cells = (long) ddom.nx * ddom.ny * ddom.nz;
@@ -3300,9 +3305,14 @@ static int mg_setup(const Coef &K)
       off[l] = tot;
       tot += ((long) mg_lev[l].sz * mg_lev[l].nz + 31) / 32 * 32;
     }
-    BB_CHECK(hipMalloc((void **) &_mg_mem, 2 * tot * sizeof(float)));
-    BB_CHECK(hipMalloc((void **) &_mg_mask, tot));
-    _mg_z = (float *) bb_grid_alloc(ddom.cc.n, sizeof(float));
+    _mg_mem = (float *) bb_try_alloc(2 * tot * sizeof(float));
+    _mg_mask = (uint8_t *) bb_try_alloc(tot);
+    _mg_z = (float *) bb_grid_try_alloc(ddom.cc.n, sizeof(float));
+    if (!_mg_mem || !_mg_mask || !_mg_z) {
+      mg_free();
+      mg_key = key;                     /* and no other try on this grid */
+      return 0;
+    }
     for (int l = 1; l < n; l++) {
       mg_r[l] = _mg_mem + off[l];
       mg_z[l] = _mg_mem + tot + off[l];

@@ -11,6 +11,7 @@ import pytest
 
 import bbconfig
 import bbhip
+from helpers import bitwise_equal
 
 pytestmark = pytest.mark.gpu
 
@@ -155,3 +156,19 @@ def test_same_step_particles(case_dir, n, walls):
     low = 4 * np.pi * a / np.prod(n) / 6
     assert velocity_difference(ref, out, n) <= \
         2 * difference_bound(out, (1., 1., 1.), low)
+
+
+def test_without_memory(case_dir):
+    """Where the levels cannot be allocated the solve keeps the Jacobi factor:
+    the bits of a solve that does not ask for them."""
+    kw = box((128, 96, 96), (1, 0, 1), (1.0, 1.0, 1.0))
+    most = ctypes.c_long.in_dll(bbhip.load(), "bb_optional_max")
+    most.value = 1 << 20                # fewer bytes than the grid's vector
+    try:
+        out = run(case_dir, kw, None, 1)
+    finally:
+        most.value = -1
+    ref = run(case_dir, kw, None, 0)
+    assert out["levels"] == 0 and out["niter"] == ref["niter"]
+    for f in ("u", "v", "w", "phi"):
+        assert bitwise_equal(out[f], ref[f]), f

@@ -118,3 +118,17 @@ def test_wait_that_gives_up(case_dir, precision):
     assert max(out["resid"]) <= 1e-8
     if precision == "PLAIN":
         same(out, ref)
+
+
+@pytest.mark.parametrize("precision", ["PLAIN", "MIXED"])
+def test_without_memory(case_dir, precision):
+    """Where the slots cannot be allocated: kernel by kernel."""
+    kw = box((64, 24, 24), (1, 0, 1), precision)
+    most = ctypes.c_long.in_dll(bbhip.load(), "bb_optional_max")
+    most.value = 0
+    try:
+        out = run(case_dir, kw, None, 1)
+    finally:
+        most.value = -1
+    assert out["tiles"][-1] == 0
+    same(out, run(case_dir, kw, None, 0))
