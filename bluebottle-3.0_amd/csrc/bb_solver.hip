@@ -2246,6 +2246,10 @@ static struct {
   double hx, hy, hz;
 } mg_key;
 static float *_mg_z = NULL, *_mg_mem = NULL;
+static double *_mg_part = NULL;        /* partials of (r, z) by workgroup of the
+                                          up kernel, of D e by tile: thin grids
+                                          have up to four times as many of the
+                                          first as of the second */
 static float *mg_r[MG_LEVELS], *mg_z[MG_LEVELS];
 static uint8_t *mg_m[MG_LEVELS];
 static uint8_t *_mg_mask = NULL;
@@ -2257,7 +2261,9 @@ static void mg_free(void)
   bb_grid_free(_mg_z);
   if (_mg_mem) BB_CHECK(hipFree(_mg_mem));
   if (_mg_mask) BB_CHECK(hipFree(_mg_mask));
+  if (_mg_part) BB_CHECK(hipFree(_mg_part));
   _mg_z = _mg_mem = NULL;
+  _mg_part = NULL;
   _mg_mask = NULL;
   mg_n = 0;
   mg_mask_of = -1;
@@ -3308,7 +3314,11 @@ static int mg_setup(const Coef &K)
     _mg_mem = (float *) bb_try_alloc(2 * tot * sizeof(float));
     _mg_mask = (uint8_t *) bb_try_alloc(tot);
     _mg_z = (float *) bb_grid_try_alloc(ddom.cc.n, sizeof(float));
-    if (!_mg_mem || !_mg_mask || !_mg_z) {
+    const long parts = mg_groups(mg_lev[0], mg_planes(mg_lev[0]));
+    const long nt = n_tiles(ddom);
+    _mg_part = (double *) bb_try_alloc((parts > nt ? parts : nt) *
+                                       sizeof(double));
+    if (!_mg_mem || !_mg_mask || !_mg_z || !_mg_part) {
       mg_free();
       mg_key = key;                     /* and no other try on this grid */
       return 0;
@@ -3418,7 +3428,7 @@ static void enqueue_iteration32(int q, bool first, const CoefT<float> &K,
   if (mg) {
     hipLaunchKernelGGL(mg_check_kernel, dim3(1), dim3(TILE_THREADS), 0,
       bb_stream, _cg_state, q - 1, _part_r, nt);
-    mg_cycle(_part_w1);
+    mg_cycle(_mg_part);
   }
   bb_kt_q = q;
   bb_kt_begin(KT_SPMV32);
@@ -3426,7 +3436,7 @@ static void enqueue_iteration32(int q, bool first, const CoefT<float> &K,
     InvMT<float> one;
     for (int i = 0; i < 27; i++) one.v[i] = 1.f;
     double *const part_r = _part_r;
-    _part_r = _part_w1;
+    _part_r = _mg_part;
     launch_group<false, float, true>(K, one, q, mg_groups(mg_lev[0],
       mg_planes(mg_lev[0])), _mg_z, pold, pnew, _Ap32);
     _part_r = part_r;
@@ -3541,8 +3551,8 @@ static void pcg_mixed(double ts, int warm)
         K.idy2*(2.*ddom.ny - (ddom.pery ? 0 : 2))*ddom.nx*ddom.nz +
         K.idz2*(2.*ddom.nz - (ddom.perz ? 0 : 2))*ddom.nx*ddom.ny;
       hipLaunchKernelGGL(mg_mean_kernel, TILES_LAUNCH, ddom, T, _e32,
-        _part_w1);
-      hipLaunchKernelGGL(mg_fold_kernel, TILES_LAUNCH, ddom, _part_w1, nt, sd,
+        _mg_part);
+      hipLaunchKernelGGL(mg_fold_kernel, TILES_LAUNCH, ddom, _mg_part, nt, sd,
         _phi, _e32);
     } else
       hipLaunchKernelGGL(mx_fold_kernel, TILES_LAUNCH, ddom, _phi, _e32);

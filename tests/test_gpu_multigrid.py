@@ -3,7 +3,7 @@
 levels take every path of the level kernels: runs of four cells and single
 ones, tiles that end inside a run, each combination of coarsened directions
 that a spacing can ask for, walls and periodic faces, a last level of more than
-4096 cells, particles."""
+4096 cells, more partials than tiles, particles."""
 import ctypes
 
 import numpy as np
@@ -84,6 +84,7 @@ def velocity_difference(a, b, n):
     ((48, 48, 512), (0, 0, 0), (1.0, 0.45, 0.2), 5),
     ((130, 96, 96), (1, 1, 1), (1.0, 1.0, 1.0), 0),
     ((100, 96, 96), (1, 0, 1), (1.0, 1.0, 1.0), 4),
+    ((64, 8, 1024), (1, 1, 1), (1.0, 8.0, 1.0), 5),
     ((64, 64, 64), (1, 1, 1), (1.0, 1.0, 1.0), 0)])
 def test_same_step(case_dir, n, per, h, levels):
     """levels: 0 where Jacobi stays (sizes with too few factors of two, no more
