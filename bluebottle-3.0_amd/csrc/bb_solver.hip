@@ -2074,8 +2074,10 @@ int bb_pcg_predict = 1;                /* 1: the first check of a sweep comes
  * loop: set by solve_begin() at the start of every solve. */
 static int solve_pass = 0;
 static int solve_step = -1;
+extern int bb_resident_last, bb_mg_last;   /* which way the last solve took */
 static void solve_begin(void)
 {
+  bb_resident_last = bb_mg_last = 0;
   if (stepnum != solve_step) {
     solve_step = stepnum;
     solve_pass = 0;
@@ -2190,13 +2192,13 @@ int bb_resident = 1;                   /* 1: grids that fit run a whole sweep
 int bb_resident_spins = 1 << 21;       /* polls (about a microsecond each)
                                           before a wait in it gives up */
 int bb_resident_last = 0;              /* tiles per workgroup of the last
-                                          sweep, 0: kernel by kernel */
+                                          solve's one-launch sweeps, 0: kernel
+                                          by kernel */
 int bb_mg = 1;                         /* 1: large grids of the mixed form
                                           without particles precondition with
                                           a V-cycle (bb_mg.h); 2: those with
                                           particles too; 0: Jacobi always */
-int bb_mg_last = 0;                    /* levels of the last mixed solve, 0:
-                                          Jacobi */
+int bb_mg_last = 0;                    /* levels of the last solve, 0: Jacobi */
 long bb_pcg_iters_total = 0;           /* PCG iterations over all solves */
 long bb_pcg_solves_total = 0;
 /* Iterations of each solve, in order (entry n % BB_SOLVE_LOG of solve n). */
@@ -2931,7 +2933,6 @@ static void enqueue_iteration(int q, const Coef &K, const InvMTab &T)
  * that sets one of those switches, times the kernels, or may not allocate. */
 static int resident_tiles(size_t esize)
 {
-  bb_resident_last = 0;
   if (!bb_resident || cg_in_scratch || bb_time_kernels) return 0;
   if (bb_spmv_variant != 3 || !bb_row_fp64 || bb_row_ry || bb_row_depth ||
       !bb_row_pairs || bb_row_zc || bb_update_variant != 1 || bb_urow_fp64 ||
@@ -3049,6 +3050,7 @@ static void pcg_plain(double ts, int warm)
   fetch_state();
   if (one_launch && cg_host->lost) {
     resident_cus = -1;
+    bb_resident_last = 0;
     one_launch = false;
     start();
     fetch_state();
@@ -3583,6 +3585,7 @@ static void pcg_mixed(double ts, int warm)
       if (cg_host->lost) {
         /* kernel by kernel from the phi of the last correction */
         resident_cus = -1;
+        bb_resident_last = 0;
         ntw = 0;
         start(1);
         fetch_state();

@@ -173,3 +173,26 @@ def test_without_memory(case_dir):
     assert out["levels"] == 0 and out["niter"] == ref["niter"]
     for f in ("u", "v", "w", "phi"):
         assert bitwise_equal(out[f], ref[f]), f
+
+
+def test_which_way(case_dir):
+    """bb_mg_last and bb_resident_last speak of the last solve alone."""
+    lib = bbhip.load()
+    levels, tiles, spins = (ctypes.c_int.in_dll(lib, "bb_" + n) for n in
+                            ("mg_last", "resident_last", "resident_spins"))
+    kw = box((128, 96, 96), (1, 0, 1), (1.0, 1.0, 1.0))
+    bbconfig.write_case(case_dir, **kw)
+    polls = spins.value
+    try:
+        with bbhip.Simulation(case_dir, kw["n"]) as s:
+            s.step()
+            assert (levels.value, tiles.value) == (4, 0)
+            lib.cuda_PP_cg_noparts()
+            assert (levels.value, tiles.value) == (0, 2)
+            lib.cuda_PP_cg_mixed()
+            assert (levels.value, tiles.value) == (4, 0)
+            spins.value = 0             # the one-launch sweep gives up
+            lib.cuda_PP_cg_noparts()
+            assert (levels.value, tiles.value) == (0, 0)
+    finally:
+        spins.value = polls
