@@ -28,6 +28,21 @@ pytestmark = pytest.mark.gpu
 FIELDS = ("u", "v", "w", "p")
 
 
+@pytest.fixture
+def kernel_by_kernel():
+    """Small grids too take the two kernels per iteration, not a sweep in one
+    launch; holds while a test runs, which checks it by one_launch()."""
+    on = ctypes.c_int.in_dll(bbhip.load(), "bb_resident")
+    saved, on.value = on.value, 0
+    yield
+    on.value = saved
+
+
+def one_launch():
+    """Whether the last solve's sweeps ran in one launch each."""
+    return ctypes.c_int.in_dll(bbhip.load(), "bb_resident_last").value > 0
+
+
 def run_mixed(case_dir, kw, nsteps, restart=0, inner_tol=None, defer=None):
     """defer: 1 pairs the inner sweep's updates of the correction, 0 updates
     it every iteration (None: library default)."""
@@ -141,7 +156,8 @@ def test_mixed_inner_tolerances(case_dir, inner_tol):
 
 
 @pytest.mark.parametrize("inner_tol", [None, 0.3])
-def test_mixed_paired_updates_same_bits(case_dir, inner_tol):
+def test_mixed_paired_updates_same_bits(case_dir, inner_tol,
+                                        kernel_by_kernel):
     """Pairing the inner sweep's updates of the correction (two terms added
     in one pass, in the same order) gives the same bits as updating it
     every iteration, across FP64 corrections (inner_tol 0.3 makes many)."""
@@ -150,6 +166,7 @@ def test_mixed_paired_updates_same_bits(case_dir, inner_tol):
     kw["hi"] = (1.3, 0.7, 1.1)
     a = run_mixed(case_dir, kw, 3, inner_tol=inner_tol, defer=0)
     b = run_mixed(case_dir, kw, 3, inner_tol=inner_tol, defer=1)
+    assert not one_launch()
     assert [st["niter"] for st in a["stats"]] == \
         [st["niter"] for st in b["stats"]]
     assert [st["nouter"] for st in a["stats"]] == \
@@ -168,13 +185,16 @@ def test_mixed_search_settings_same_bits(case_dir):
     kw = bbconfig.channel(n=(64, 32, 128))
     out = []
     for tzb32, nts32 in ((1, 1), (3, 0), (8, 0)):
+        ctypes.c_int.in_dll(lib, "bb_spmv_variant").value = 2
         ctypes.c_int.in_dll(lib, "bb_spmv_tzb32").value = tzb32
         ctypes.c_int.in_dll(lib, "bb_spmv_nts32").value = nts32
         try:
             out.append(run_mixed(case_dir, kw, 2))
         finally:
+            ctypes.c_int.in_dll(lib, "bb_spmv_variant").value = 3
             ctypes.c_int.in_dll(lib, "bb_spmv_tzb32").value = 0
             ctypes.c_int.in_dll(lib, "bb_spmv_nts32").value = 1
+        assert ctypes.c_int.in_dll(lib, "bb_spmv_last").value == 2
     for res in out[1:]:
         assert [st["niter"] for st in res["stats"]] == \
             [st["niter"] for st in out[0]["stats"]]
@@ -182,21 +202,27 @@ def test_mixed_search_settings_same_bits(case_dir):
             assert np.array_equal(res["gpu"][f], out[0]["gpu"][f]), f
 
 
-@pytest.mark.parametrize("precision", ["PLAIN", "MIXED"])
-def test_predicted_checks_same_bits(case_dir, precision):
+@pytest.mark.parametrize("precision,n,mg", [
+    ("PLAIN", (32, 32, 32), 1), ("MIXED", (32, 32, 32), 1),
+    ("MIXED", (80, 64, 64), 2)])
+def test_predicted_checks_same_bits(case_dir, precision, n, mg,
+                                    kernel_by_kernel):
     """The host's first check of a PCG sweep after 0.8 of the length the
-    same sweep had one timestep earlier (bb_pcg_predict) only moves the
-    points where the host reads the CG state: sedimentation 32^3 with two
-    spheres over three timesteps (several Lamb passes each) gives the same
-    iterations and the same bits with and without it."""
+    same sweep had one timestep earlier (bb_pcg_predict), or after all of
+    it where the sweep is preconditioned with a V-cycle (80 x 64 x 64 with
+    bb_mg = 2), only moves the points where the host reads the CG state:
+    sedimentation with two spheres over three timesteps (several Lamb passes
+    each) gives the same iterations and the same bits with and without it."""
     lib = bbhip.load()
-    kw, parts = bbconfig.sediment(n=(32, 32, 32), nparts=2, a=4.0, seed=11)
+    kw, parts = bbconfig.sediment(n=n, nparts=2, a=4.0, seed=11)
     kw["extensions"] = dict(kw.get("extensions") or {},
                             pp_precision=precision)
     knob = ctypes.c_int.in_dll(lib, "bb_pcg_predict")
-    saved = knob.value
+    cycle = ctypes.c_int.in_dll(lib, "bb_mg")
+    saved = knob.value, cycle.value
     out = []
     try:
+        cycle.value = mg
         for pred in (0, 1):
             knob.value = pred
             bbconfig.write_case(case_dir, **kw)
@@ -206,12 +232,15 @@ def test_predicted_checks_same_bits(case_dir, precision):
                 for _ in range(3):
                     s.step()
                     res["iters"].append(s.pp_stats()["niter"])
+                    assert not one_launch()
+                    assert (ctypes.c_int.in_dll(lib, "bb_mg_last").value
+                            > 0) == (mg == 2)
                 s.pull()
                 for f in FIELDS:
                     res["f"][f] = np.array(s.field(f))
             out.append(res)
     finally:
-        knob.value = saved
+        knob.value, cycle.value = saved
     print("iterations (last solve of each step):", out[0]["iters"],
           out[1]["iters"])
     assert out[0]["iters"] == out[1]["iters"]

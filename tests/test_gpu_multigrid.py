@@ -159,6 +159,89 @@ def test_same_step_particles(case_dir, n, walls):
         2 * difference_bound(out, (1., 1., 1.), low)
 
 
+def test_steps_with_moving_particles(case_dir):
+    """Three timesteps with spheres that move by part of a cell in each: the
+    levels' masks follow, and the same bits come out where the solver's buffers
+    are freed before each step (void bb_solver_free(void)), which builds the
+    levels anew."""
+    lib = bbhip.load()
+    on = ctypes.c_int.in_dll(lib, "bb_mg")
+    free = getattr(lib, "_Z14bb_solver_freev")
+    kw, parts = bbconfig.sediment(n=(80, 64, 64), nparts=2, a=8.0, seed=13)
+    for P, c, v in zip(parts, ((20., 20., 20.), (60., 40., 45.)), (0.3, -0.3)):
+        P.update(x=c[0], y=c[1], z=c[2], u=v, w=v)
+    kw["extensions"] = {"pp_precision": "MIXED"}
+    out, saved = [], on.value
+    on.value = 2
+    try:
+        for anew in (0, 1):
+            bbconfig.write_case(case_dir, **kw)
+            bbconfig.write_parts(case_dir, parts)
+            with bbhip.Simulation(case_dir, kw["n"]) as s:
+                steps, phase = [], []
+                for _ in range(3):
+                    if anew:
+                        s.sync()
+                        free()
+                    s.step()
+                    st = s.pp_stats()
+                    assert ctypes.c_int.in_dll(lib, "bb_mg_last").value == 4
+                    assert st["resid"] <= 1e-8 and st["niter"] <= 30
+                    s.pull()
+                    phase.append(np.array(s.field("phase")) >= 0)
+                    steps.append({f: np.array(s.field(f))
+                                  for f in ("u", "v", "w", "phi")})
+                    steps[-1]["niter"] = st["niter"]
+                assert all((a != b).any() for a, b in zip(phase, phase[1:]))
+            out.append(steps)
+    finally:
+        on.value = saved
+    for a, b in zip(*out):
+        assert a["niter"] == b["niter"]
+        for f in ("u", "v", "w", "phi"):
+            assert bitwise_equal(a[f], b[f]), f
+
+
+def test_steps_warm_start(case_dir):
+    """Three timesteps from earlier solutions (the guess without its network)
+    with the V-cycle and with the Jacobi factor.  Each solve leaves a velocity
+    difference B (difference_bound) and one in dt / rho grad p, which the next
+    steps start from: n B of the n steps before, so 1 + 2 + 3 B after three
+    (seven: convection and diffusion change it by less than a sixth)."""
+    lib = bbhip.load()
+    h = (1.0, 1.0, 1.0)
+    kw = box((128, 96, 96), (1, 1, 1), h)
+    kw["extensions"]["pp_warmstart"] = "LEARNED"
+    on = ctypes.c_int.in_dll(lib, "bb_mg")
+    net = ctypes.c_int.in_dll(lib, "bb_warm_use_net")
+    saved = on.value, net.value
+    net.value = 0
+    out = []
+    try:
+        for mg in (0, 1):
+            on.value = mg
+            bbconfig.write_case(case_dir, **kw)
+            with bbhip.Simulation(case_dir, kw["n"]) as s:
+                stats = []
+                for _ in range(3):
+                    s.step()
+                    stats.append(s.pp_stats())
+                    assert stats[-1]["resid"] <= 1e-8
+                assert ctypes.c_int.in_dll(lib, "bb_mg_last").value == 4 * mg
+                s.pull()
+                out.append({f: np.array(s.field(f)) for f in "uvw"})
+                out[-1].update(dt=s.scalar("dt"), n=[t["niter"] for t in stats],
+                               sp_rhs=max(t["sp_rhs"] for t in stats))
+    finally:
+        on.value, net.value = saved
+    ref, got = out
+    print("iterations", ref["n"], got["n"])
+    assert max(got["n"]) <= 30 < ref["n"][0] and got["n"][-1] < got["n"][0]
+    low = min((2 - 2 * np.cos(2 * np.pi / m)) for m in kw["n"]) / 6
+    assert velocity_difference(ref, got, kw["n"]) <= \
+        7 * difference_bound(got, h, low)
+
+
 def test_without_memory(case_dir):
     """Where the levels cannot be allocated the solve keeps the Jacobi factor:
     the bits of a solve that does not ask for them."""

@@ -25,10 +25,12 @@ def set_knobs(variant=3, tzb=0, batch=16, defer=0):
     allows it, else as 2; 2: over z-columns of tzb tiles (0: automatic);
     0: direct neighbour loads (the cross-check implementation); defer = 1:
     phi updated every second iteration with both terms (odd iterations
-    leave it)."""
+    leave it).  variant 4: a whole sweep in one launch (the library's choice
+    on a grid that fits, with every other setting at its default)."""
     lib = bbhip.load()
+    ctypes.c_int.in_dll(lib, "bb_resident").value = variant == 4
     ctypes.c_int.in_dll(lib, "bb_defer_phi").value = defer
-    ctypes.c_int.in_dll(lib, "bb_spmv_variant").value = variant
+    ctypes.c_int.in_dll(lib, "bb_spmv_variant").value = min(variant, 3)
     ctypes.c_int.in_dll(lib, "bb_spmv_tzb").value = tzb
     ctypes.c_int.in_dll(lib, "bb_pcg_batch").value = batch
 
@@ -38,7 +40,7 @@ def default_knobs():
     """Each test sets its knobs; the library keeps them, so put the
     defaults back for the tests that follow."""
     yield
-    set_knobs(defer=1)
+    set_knobs(4, defer=1)
 
 
 def run_pair(case_dir, kw, nsteps, variant=3, tzb=0, batch=16, defer=0):
@@ -60,6 +62,8 @@ def run_pair(case_dir, kw, nsteps, variant=3, tzb=0, batch=16, defer=0):
         for f in FIELDS:
             out["gpu"][f] = np.array(s.field(f))
         out["gpu_dt"] = s.scalar("dt")
+    one_launch = ctypes.c_int.in_dll(bbhip.load(), "bb_resident_last").value
+    assert (one_launch > 0) == (variant == 4)
     return out
 
 
@@ -104,7 +108,8 @@ def test_channel_small(case_dir):
 
 @pytest.mark.parametrize("variant,tzb,defer",
                          [(0, 0, 0), (2, 1, 0), (2, 4, 0), (2, 4, 1),
-                          (2, 1, 1), (2, 8, 1), (3, 0, 0), (3, 0, 1)])
+                          (2, 1, 1), (2, 8, 1), (3, 0, 0), (3, 0, 1),
+                          (4, 0, 1)])
 def test_channel_bitwise(case_dir, variant, tzb, defer):
     out = run_pair(case_dir, bbconfig.channel(n=(64, 32, 32)), 3, variant,
                    tzb, defer=defer)
@@ -117,7 +122,7 @@ def test_channel_bitwise(case_dir, variant, tzb, defer):
                          [(0, 0, 16, 0), (0, 0, 5, 0), (2, 2, 1, 0),
                           (2, 4, 5, 0), (2, 3, 16, 0), (2, 2, 1, 1),
                           (2, 4, 5, 1), (2, 3, 16, 1), (2, 8, 16, 1),
-                          (3, 0, 16, 0), (3, 0, 5, 1)])
+                          (3, 0, 16, 0), (3, 0, 5, 1), (4, 0, 16, 1)])
 def test_ragged_sizes(case_dir, variant, tzb, batch, defer):
     """x not a multiple of the 64-lane wavefront, y not a multiple of the
     row group, z not a multiple of the tile depth (and the tile count in z,
@@ -160,7 +165,7 @@ def test_periodic_all_and_wide_x(case_dir):
 
 
 @pytest.mark.parametrize("variant,defer", [(2, 0), (0, 0), (2, 1), (3, 0),
-                                           (3, 1)])
+                                           (3, 1), (4, 1)])
 def test_periodic_all_25d(case_dir, variant, defer):
     per = ("PERIODIC",)
     vel = {c: {f: per for f in "WESNBT"} for c in "uvw"}
@@ -169,7 +174,8 @@ def test_periodic_all_25d(case_dir, variant, defer):
               pp_residual=1e-8, p_bc={f: per for f in "WESNBT"}, vel_bc=vel,
               init_cond="QUIESCENT",
               extensions={"fixed_dt": 1e-3, "perturb": (6, 0.2)})
-    out = run_pair(case_dir, kw, 3, variant=variant, tzb=2, defer=defer)
+    out = run_pair(case_dir, kw, 3, variant=variant,
+                   tzb=0 if variant == 4 else 2, defer=defer)
     for f in FIELDS:
         assert bitwise_equal(out["gpu"][f], out["orc"][f]), \
             describe(f, out["gpu"][f], out["orc"][f])

@@ -107,6 +107,24 @@ def test_one_launch_particles_same_bits(case_dir, n, walls, precision):
 
 
 @pytest.mark.parametrize("precision", ["PLAIN", "MIXED"])
+def test_one_launch_warm_start_same_bits(case_dir, precision):
+    """From earlier solutions instead of phi = 0 (the guess without its
+    network)."""
+    kw, parts = bbconfig.sediment(n=(64, 32, 48), nparts=2, a=5.0, seed=13)
+    kw["extensions"] = {"pp_precision": precision, "pp_warmstart": "LEARNED"}
+    net = ctypes.c_int.in_dll(bbhip.load(), "bb_warm_use_net")
+    saved, net.value = net.value, 0
+    try:
+        ref = run(case_dir, kw, parts, 0, nsteps=3)
+        out = run(case_dir, kw, parts, 1, nsteps=3)
+    finally:
+        net.value = saved
+    assert out["tiles"][-1] > 0 and ref["tiles"][-1] == 0
+    assert out["iters"][-1] < out["iters"][0]
+    same(out, ref)
+
+
+@pytest.mark.parametrize("precision", ["PLAIN", "MIXED"])
 def test_wait_that_gives_up(case_dir, precision):
     """With no poll allowed the sweep gives up at its first meeting and the
     solve runs kernel by kernel: the same bits for the plain form, the same
