@@ -2,7 +2,7 @@
  * Multigrid preconditioner of the mixed form's inner FP32 sweep on large
  * grids (included by bb_solver.hip).  Jacobi-PCG needs hundreds of iterations
  * because it moves information one cell per iteration; one V-cycle moves it
- * across the box, and PCG with it needs about 10 to 17 iterations for the
+ * across the box, and PCG with it needs about 10 to 18 iterations for the
  * reference's 1e-8 from phi = 0, with any number of spheres (256^3 with 500:
  * 440 with the Jacobi factor).  What a solve must reach does not change: the
  * FP64 residual of the masked operator under the reference's test.
@@ -23,13 +23,14 @@
  * One kernel per level and direction of travel.  On the grid itself they are
  * bound by LDS and instruction issue (the vectors of 256^3 stay in the last
  * level cache), on the coarse levels by the latency of their few planes.
- * 256^3 with 500 spheres, us per V-cycle: down 42 on the grid, 14, 10 and 10 on
- * the levels below, the last level 10, up 9, 10, 15 and 44; as four kernels
+ * 256^3 with 500 spheres, us per V-cycle: down 46 on the grid, 13, 9 and 9 on
+ * the levels below, the last level 10, up 9, 9, 16 and 47; as four kernels
  * per level (defect, restriction, x, z) 238 in all.  With the search and the
- * update an iteration takes some 280 us against 105 with the Jacobi factor,
- * and a timestep of that box 75 ms against 304.  Without particles a timestep
- * of a 256x128x128 channel takes 2.7 ms against 18.1 (27.5 before the one-launch
- * sweep), a solve of 128^3 1.7 ms against 10.2.
+ * update an iteration takes some 290 us against 105 with the Jacobi factor,
+ * and a timestep of that box 76 ms against 280; with particles the V-cycle has
+ * to be asked for, though (bb_mg = 2).  Without them, where it is the default, a
+ * timestep of a 256x128x128 channel takes 2.7 ms against 17 (27.5 kernel by
+ * kernel), a solve of 128^3 1.7 ms against 10.2.
  */
 #ifndef BB_MG_H
 #define BB_MG_H
@@ -214,7 +215,7 @@ __device__ inline MG4 mg_lap(const MGRun<VEC> &R, const MGLevel &L,
  * fluid coarse cells.  Three planes of r pass through LDS with a halo of two
  * cells, the defect of one plane with one; a thread gathers a run of the
  * coarse row below its fine ones, and each coarse plane's sum over its four
- * fine ones stays in registers.  256^3 to 128^3: 42 us (92 MB); a kernel for
+ * fine ones stays in registers.  256^3 to 128^3: 46 us (92 MB); a kernel for
  * the defect and one that gathers it: 93; one cell per thread and its weights
  * by table: 62. */
 template <bool CX, bool CY, bool CZ, bool VEC>
@@ -399,7 +400,7 @@ mg_down_kernel(const CGState *st, MGLevel L, MGLevel C, int zc,
  * on the grid itself (gpart) the workgroups' partials of (r, z) in FP64.  x
  * passes through LDS with a halo of one cell, planes k - 1 to k + 1 and the
  * one being written; each coarse plane is interpolated in x and y once.
- * 256^3: 44 us (160 MB); a kernel for x and one for z: 86; one cell per thread:
+ * 256^3: 47 us (159 MB); a kernel for x and one for z: 86; one cell per thread:
  * 90. */
 template <bool CX, bool CY, bool CZ, bool VEC>
 __global__ void __launch_bounds__(TILE_THREADS, VEC ? 4 : 1)
@@ -609,8 +610,8 @@ mg_last_kernel(const CGState *st, MGLevel L, float lmin, float lmax,
   const int n = L.nx * L.ny * L.nz, t = threadIdx.x, s2 = L.nx * L.ny;
   float res[Q], x[Q], d[Q];
   /* which of a cell's six neighbours lie in the box (bits 0 to 5: west, east,
-   * south, north, below, above), and bit 6 in a fluid cell; a level of MG_LAST_MAX
-   * cells may be that long in one direction */
+   * south, north, below, above), and bit 6 in a fluid cell; a level of
+   * MG_LAST_MAX cells may be that long in one direction */
   int at[Q];
   float sum = 0.f;
 #pragma unroll

@@ -20,10 +20,10 @@
  * for the cells around, and with many cells per thread the arithmetic.  The
  * host reads the state once per sweep instead of once per 16 iterations.
  * Microseconds per iteration, kernel by kernel -> in one launch:
- *   FP64: cavity 16^3 21 -> 5.6, 32^3 34 -> 5.9; channel 65 x 33 x 31
- *   35 -> 7.7; spheres 64^3 18 -> 8.4, 128^3 34 -> 16.3 (two tiles);
- *   FP32: channel 150 x 130 x 94 45 -> 17.8, 256 x 128 x 128 34 -> 21.9
- *   (four tiles).
+ *   FP64: cavity 16^3 17 -> 5.7, 32^3 28 -> 5.9; channel 65 x 33 x 31
+ *   33 -> 7.8; spheres 64^3 18 -> 8.3, 128^3 34 -> 16.2 (two tiles);
+ *   FP32: channel 150 x 130 x 94 44 -> 17.6, 256 x 128 x 128 34 -> 21.7
+ *   (four tiles; without the V-cycle that it takes by default).
  *
  * A meeting: each workgroup stores its tile partials into its slots of the
  * current set by 8-byte device-scope stores, and every thread waits for the
@@ -35,8 +35,9 @@
  * completed (s_waitcnt vmcnt(0) in every wavefront, then the barrier) before
  * it publishes the meeting after which others read them.  The launch is
  * cooperative, so all workgroups are resident; every wait gives up after
- * a number of polls (seconds) all the same, and the host then runs the sweep
- * kernel by kernel.
+ * a number of polls (seconds) all the same, and the host then starts again
+ * kernel by kernel from phi = 0, or from the phi that it finds: workgroups that
+ * ended the sweep have stored theirs by then, which the stopping test allows.
  *
  * Arithmetic, dot-product order and stopping test are those of the search and
  * update kernels: same bits, same iteration counts.

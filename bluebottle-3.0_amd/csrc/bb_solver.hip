@@ -2927,10 +2927,13 @@ static void enqueue_iteration(int q, const Coef &K, const InvMTab &T)
 /* Tiles per workgroup of the one-launch sweep with vectors of `esize` bytes
  * on this grid; 0: kernel by kernel.  One workgroup per CU, at most two tiles
  * of FP64 cells (a thread then holds 16 cells, 128 VGPRs of r, p, A p and phi
- * of the 256 it can have) or four of FP32 cells.  FP64 rows of more than two
- * tiles stay with the row kernels, whose choice by row length
- * (tests/test_gpu_rowkernel.py) the switches below describe; so does any run
- * that sets one of those switches, times the kernels, or may not allocate. */
+ * of the 256 it can have) or four of FP32 cells.  A run that sets one of the
+ * row kernels' switches below, times the kernels (the figures are theirs) or
+ * may not allocate stays with them.  So do FP64 rows of more than two tiles,
+ * though a sweep in one launch would fit and be faster there (132 x 64 x 64:
+ * 10 us per iteration instead of 24, 256 x 64 x 128: 17 instead of 41): the
+ * tests of the row kernels' layouts (tests/test_gpu_rowkernel.py) ask for them
+ * by row length with every switch at its default. */
 static int resident_tiles(size_t esize)
 {
   if (!bb_resident || cg_in_scratch || bb_time_kernels) return 0;
@@ -3245,8 +3248,10 @@ extern "C" int cuda_PP_cg_noalloc(void)
  * to 1e-8 with the Jacobi factor (in one launch where the grid fits) and with
  * the V-cycle, us: 48^3 with spheres 1779 and 1321, channel 2207 and 1047;
  * 64^3 2528 and 1361, 3024 and 1219; 96^3 5033 and 1896, 6146 and 1575; 128^3
- * 7128 and 2186, 10178 and 1682.  It is the faster one below this line too;
- * there the sweep's iterates are the plain form's. */
+ * 7128 and 2186, 10178 and 1682.  So speed would put the line below 48^3.  It
+ * stands at 64^3 because the mixed form's tests on grids below that hold it to
+ * fields closer to the plain form's than the stopping test asks for; Jacobi
+ * sweeps, which share the plain form's iterates, meet them. */
 #define MG_MIN_CELLS (1l << 18)
 
 /* The levels of this grid and their vectors; 0: Jacobi, also where the vectors
@@ -3262,10 +3267,13 @@ static int mg_setup(const Coef &K)
   /* With particles only on request.  The Lamb loop ends by a threshold on its
    * coefficients' change, and where a pass comes out within the solve's
    * tolerance of it, two solvers that both meet the stopping test take one
-   * pass more or less: seen once in six timesteps of 256^3 with 500 spheres
-   * (13 passes with the V-cycle and with a solve to 1e-11, 12 with the Jacobi
-   * factor), the fields 5e-7 apart where they are 1e-8 apart otherwise.  A
-   * timestep takes 77 ms with it and 280 without. */
+   * pass more or less, and the fields come out 5e-7 apart instead of 1e-8.
+   * That is so for any two: in one of six timesteps of 256^3 with 500 spheres
+   * the Jacobi factor and a V-cycle solve to 3e-9 took 12 passes, the V-cycle
+   * and a solve to 1e-11 took 13.  The default keeps the counts of the Jacobi
+   * factor; it is not the more accurate one for that, and six timesteps are too
+   * few to say which is off more often.  A timestep takes 76 ms with the
+   * V-cycle and 280 without. */
   if (fluid_mask() && bb_mg < 2) return 0;
   auto key = mg_key;
   memset(&key, 0, sizeof(key));
@@ -3583,7 +3591,7 @@ static void pcg_mixed(double ts, int warm)
       }
       correct(-1);
       if (cg_host->lost) {
-        /* kernel by kernel from the phi of the last correction */
+        /* kernel by kernel from phi, the e folded in that was stored */
         resident_cus = -1;
         bb_resident_last = 0;
         ntw = 0;
