@@ -83,10 +83,11 @@ static Grid make_grid(const grid_info &G)
 static struct { void *user, *raw; } grid_tab[GRID_ALLOCS];
 
 /* Buffers that only make a solve faster, and that it does without where they
- * do not fit: NULL instead of an exit.  They come in the first solve, before
- * the arrays of the learned guess (nine of the grid in FP64 and the network's),
- * and one may take 1/32 of the free memory, so that a run that fits without
- * them still does. */
+ * do not fit: NULL instead of an exit.  They come in the first solve.  Where
+ * the learned guess allocates after that (the solutions of earlier solves and
+ * of the last timesteps' Lamb passes, some thirty FP64 arrays of the grid), one
+ * may take 1/64 of the free memory, a grid array in FP32 being the largest, so
+ * that a run that fits without them still does; elsewhere half of it. */
 long bb_optional_max = -1;             /* bytes of one at most; -1: only the
                                           bound above */
 
@@ -96,7 +97,7 @@ void *bb_try_alloc(size_t bytes)
   size_t left = 0, all = 0;
   if (bb_optional_max >= 0 && bytes > (size_t) bb_optional_max) return NULL;
   BB_CHECK(hipMemGetInfo(&left, &all));
-  if (bytes > left / 32) return NULL;
+  if (bytes > left / (pp_warmstart == PP_WARM_LEARNED ? 64 : 2)) return NULL;
   hipError_t e = hipMalloc(&p, bytes);
   if (e == hipSuccess) return p;
   (void) hipGetLastError();
